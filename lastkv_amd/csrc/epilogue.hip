@@ -617,56 +617,82 @@ struct BlendParams {
   int32_t d_npages;
 };
 
-// One thread per 8-element (16-byte) run of one block of one (layer, sequence, head).  K and
-// V runs are handled by separate threads (kind = item parity).
+// One workgroup per (K or V, 32-token block, kv head, sequence, group of kBlendLayers layers): thread t
+// holds the block's 16-byte runs t and t + 256.  Bound by HBM (the rings are read and written once, the
+// shared block is read once per layer group).  The indices are uniform over the workgroup, so they cost
+// scalar work only, and every load of the group's layers is issued before the first use.
+constexpr int kBlendLayers = 4;
+constexpr int kBlendRuns = kBlockElems / 8 / 256;
+
+// ring := bf16(bf16(a * bf16(deep * s)) + bf16(om * ring)) for one value (s is 1 for K: exact).
+__device__ inline float blend_value(float deep, float own, float a, float om, float s) {
+  return rb(a * rb(deep * s)) + rb(om * own);  // (rounded by the packing)
+}
+
 __global__ __launch_bounds__(256) void blend_kernel(const BlendParams p) {
-  const int64_t per_block = kBlockElems / 8;
-  const int64_t total = static_cast<int64_t>(p.layers) * p.batch * p.heads * p.nblk * per_block * 2;
-  for (int64_t item = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; item < total;
-       item += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+  const int groups = (p.layers + kBlendLayers - 1) / kBlendLayers;
+  const int64_t total = static_cast<int64_t>(groups) * p.batch * p.heads * p.nblk * 2;
+  for (int64_t item = blockIdx.x; item < total; item += gridDim.x) {
     const int kind = static_cast<int>(item & 1);
     int64_t rest = item >> 1;
-    const int run = static_cast<int>(rest % per_block);
-    rest /= per_block;
     const int blk = p.blk0 + static_cast<int>(rest % p.nblk);
     rest /= p.nblk;
     const int g = static_cast<int>(rest % p.heads);
     rest /= p.heads;
     const int b = static_cast<int>(rest % p.batch);
-    const int l = static_cast<int>(rest / p.batch);
-    const int off = run * 8;
+    const int l0 = static_cast<int>(rest / p.batch) * kBlendLayers;
     const int base_tok = blk * kBlockTokens;
     const int ring_blk = (base_tok % p.ring_tokens) >> 5;
-    const int lh = l * p.heads + g;
-    const float a = p.alpha[lh], om = p.om[lh];
-    const float s = (kind == 1 && p.vs != nullptr) ? p.vs[lh] : 1.f;
-    const int64_t doff = (p.d_tab ? 0 : b * p.d_ss) + g * p.d_hs +
-                         write_block(p.d_tab, p.d_tab_stride, p.d_page, p.d_npages, b, blk);
-    const int64_t roff = p.r_tab ? g * p.r_hs + write_block(p.r_tab + l * p.r_tab_ls, p.r_tab_stride, p.r_page,
-                                                            p.r_npages, b, ring_blk)
-                                 : l * p.r_ls + b * p.r_ss + g * p.r_hs + static_cast<int64_t>(ring_blk) * kBlockElems;
-    const uint16_t* dsrc = (kind == 0 ? p.dk : p.dv) + doff + off;
-    uint16_t* rdst = (kind == 0 ? p.rk : p.rv) + roff + off;
-    const uint4 dv4 = *reinterpret_cast<const uint4*>(dsrc);
-    uint4 rv4 = *reinterpret_cast<const uint4*>(rdst);
-    const uint16_t* de = reinterpret_cast<const uint16_t*>(&dv4);
-    uint16_t* re = reinterpret_cast<uint16_t*>(&rv4);
-    // token index of each element of the run: K runs hold 8 dims of one token, V runs 8 tokens
-    int w_k = 0;
-    if (kind == 0) {
-      const int r = (off >> 5) & 15, u = (off >> 11) & 1;
-      w_k = 8 * (r >> 2) + 4 * u + (r & 3);
-    }
+    const uint16_t* dsrc = (kind == 0 ? p.dk : p.dv) + (p.d_tab ? 0 : b * p.d_ss) + g * p.d_hs +
+                           write_block(p.d_tab, p.d_tab_stride, p.d_page, p.d_npages, b, blk);
+    uint16_t* rdst[kBlendLayers];
+    uint4 d[kBlendRuns], r[kBlendLayers][kBlendRuns];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int tokpos = base_tok + (kind == 0 ? w_k : ((off & 31) + j));
-      if (tokpos < p.start || tokpos >= p.end) continue;
-      const float src = bf16_bits_to_f32(de[j]);
-      const float own = bf16_bits_to_f32(re[j]);
-      const float scaled = kind == 1 ? rb(src * s) : src;
-      re[j] = f32_to_bf16_bits(rb(a * scaled) + rb(om * own));
+    for (int i = 0; i < kBlendRuns; ++i) d[i] = *reinterpret_cast<const uint4*>(dsrc + (threadIdx.x + 256 * i) * 8);
+#pragma unroll
+    for (int j = 0; j < kBlendLayers; ++j) {
+      const int l = min(l0 + j, p.layers - 1);  // (past the last layer: reread, not written)
+      rdst[j] = (kind == 0 ? p.rk : p.rv) +
+                (p.r_tab ? g * p.r_hs + write_block(p.r_tab + l * p.r_tab_ls, p.r_tab_stride, p.r_page, p.r_npages, b, ring_blk)
+                         : l * p.r_ls + b * p.r_ss + g * p.r_hs + static_cast<int64_t>(ring_blk) * kBlockElems);
+#pragma unroll
+      for (int i = 0; i < kBlendRuns; ++i) r[j][i] = load_nt(rdst[j] + (threadIdx.x + 256 * i) * 8);
     }
-    *reinterpret_cast<uint4*>(rdst) = rv4;
+    const bool whole = base_tok >= p.start && base_tok + kBlockTokens <= p.end;  // (uniform)
+#pragma unroll
+    for (int j = 0; j < kBlendLayers; ++j) {
+      const int l = l0 + j;
+      if (l >= p.layers) break;
+      const int lh = l * p.heads + g;
+      const float a = p.alpha[lh], om = p.om[lh];
+      const float s = (kind == 1 && p.vs != nullptr) ? p.vs[lh] : 1.f;
+#pragma unroll
+      for (int i = 0; i < kBlendRuns; ++i) {
+        const int off = (threadIdx.x + 256 * i) * 8;
+        float dv[8], own[8];
+        unpack8(d[i], dv);
+        unpack8(r[j][i], own);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dv[e] = blend_value(dv[e], own[e], a, om, s);
+        uint4 n = pack8(dv);
+        if (!whole) {  // a block at the chunk's edge keeps the other tokens' bits
+          // K runs hold 8 dims of one token, V runs 8 tokens
+          const int tr = (off >> 5) & 15, u = (off >> 11) & 1;
+          const int w_k = 8 * (tr >> 2) + 4 * u + (tr & 3);
+          auto pick = [&](uint32_t now, uint32_t old, int e) {
+            uint32_t m = 0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int tok = base_tok + (kind == 0 ? w_k : (off & 31) + e + h);
+              if (tok >= p.start && tok < p.end) m |= 0xffffu << (16 * h);
+            }
+            return (now & m) | (old & ~m);
+          };
+          n = make_uint4(pick(n.x, r[j][i].x, 0), pick(n.y, r[j][i].y, 2), pick(n.z, r[j][i].z, 4), pick(n.w, r[j][i].w, 6));
+        }
+        store_nt(rdst[j] + off, n);
+      }
+    }
   }
 }
 
@@ -856,9 +882,7 @@ extern "C" int32_t lkv_blend_chunk(const lkv_blend_args* a, lkv_stream_t stream)
   p.d_tab_stride = a->deep_table_stride;
   p.d_page = a->deep_page_stride;
   p.d_npages = a->deep_num_pages;
-  const int64_t total = static_cast<int64_t>(a->layers) * a->batch * a->kv_heads * p.nblk * (kBlockElems / 8) * 2;
-  const int64_t want = (total + 255) / 256;
-  const int grid = static_cast<int>(want < 65536 ? want : 65536);
-  blend_kernel<<<grid, 256, 0, as_stream(stream)>>>(p);
+  const int64_t items = static_cast<int64_t>((a->layers + kBlendLayers - 1) / kBlendLayers) * a->batch * a->kv_heads * p.nblk * 2;
+  blend_kernel<<<static_cast<unsigned>(std::min<int64_t>(items, 1 << 30)), 256, 0, as_stream(stream)>>>(p);
   return check_launch("lkv_blend_chunk");
 }

@@ -2,6 +2,8 @@
 // layers of the serving path (the roles of vLLM's fused_add_rms_norm and silu_and_mul around the
 // attention backend).  Both keep the rounding points of the torch expressions they replace, so a
 // row computed here differs from torch's only where torch's own reduction order would.
+#include <algorithm>
+
 #include "common.h"
 #include "runtime.h"
 
@@ -10,7 +12,7 @@ namespace {
 
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxHidden = 16384;  // 8 chunks of 8 elements per thread
-constexpr int kNormChunks = kNormMaxHidden / (kNormThreads * 8);
+constexpr int kNormMaxChunks = kNormMaxHidden / (kNormThreads * 8);
 
 struct NormParams {
   const uint16_t* x;
@@ -39,35 +41,47 @@ __device__ inline uint4 pack8(const float (&f)[8]) {
   return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7]));
 }
 
-// One workgroup per row; thread t owns the 8-element chunks t, t + 256, ...  With kAdd the row is
-// residual := bf16(residual + x) first (torch's bf16 add) and the normalised row is that sum.
+// One workgroup per row; thread t owns the 8-element chunks t, t + 256, ... (kChunks of them).  With kAdd
+// the row is residual := bf16(residual + x) first (torch's bf16 add) and the normalised row is that sum.
 // Then, as transformers' LlamaRMSNorm: h = float(row); r = rsqrt(sum(h^2) * (1 / hidden) + eps);
 // out = bf16(w * bf16(h * r)).
-template <bool kAdd>
+// Bound by HBM: every load (x, residual and the weights) is issued before the first use, with no branch
+// between them (a chunk past the row rereads the last one), so a row costs one memory round trip.
+template <bool kAdd, int kChunks>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const NormParams p) {
   __shared__ float part[kNormThreads / 64];
   const int row = blockIdx.x;
   const int chunks = p.hidden >> 3;
   const uint4* x = reinterpret_cast<const uint4*>(p.x + row * p.x_stride);
   uint4* res = kAdd ? reinterpret_cast<uint4*>(p.residual + row * p.res_stride) : nullptr;
-  float v[kNormChunks][8];
+  const uint4* w = reinterpret_cast<const uint4*>(p.w);
+  uint4 xv[kChunks], rv[kChunks], wv[kChunks];
+#pragma unroll
+  for (int k = 0; k < kChunks; ++k) {
+    const int c = min(static_cast<int>(threadIdx.x) + k * kNormThreads, chunks - 1);
+    xv[k] = load_nt(x + c);
+    if (kAdd) rv[k] = res[c];
+  }
+#pragma unroll
+  for (int k = 0; k < kChunks; ++k) wv[k] = w[min(static_cast<int>(threadIdx.x) + k * kNormThreads, chunks - 1)];
   float ss = 0.f;
 #pragma unroll
-  for (int k = 0; k < kNormChunks; ++k) {
+  for (int k = 0; k < kChunks; ++k) {
     const int c = threadIdx.x + k * kNormThreads;
     if (c < chunks) {
-      unpack8(x[c], v[k]);
+      float v[8];
+      unpack8(xv[k], v);
       if (kAdd) {
         float r[8];
-        unpack8(res[c], r);
+        unpack8(rv[k], r);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) r[j] += v[k][j];
-        const uint4 s = pack8(r);
-        res[c] = s;
-        unpack8(s, v[k]);
+        for (int j = 0; j < 8; ++j) r[j] += v[j];
+        xv[k] = pack8(r);
+        res[c] = xv[k];
+        unpack8(xv[k], v);
       }
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(v[k][j], v[k][j], ss);
+      for (int j = 0; j < 8; ++j) ss = __builtin_fmaf(v[j], v[j], ss);
     }
   }
   // row sum: within the wave (DPP through the shuffle builtins), then across the 4 waves
@@ -77,17 +91,17 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const NormParams 
   __syncthreads();
   const float total = (part[0] + part[1]) + (part[2] + part[3]);
   const float r = rsqrtf(total * (1.f / static_cast<float>(p.hidden)) + p.eps);
-  const uint4* w = reinterpret_cast<const uint4*>(p.w);
   uint4* out = reinterpret_cast<uint4*>(p.out + row * p.out_stride);
 #pragma unroll
-  for (int k = 0; k < kNormChunks; ++k) {
+  for (int k = 0; k < kChunks; ++k) {
     const int c = threadIdx.x + k * kNormThreads;
     if (c < chunks) {
       float h[8], wf[8];
+      unpack8(xv[k], h);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) h[j] = v[k][j] * r;
+      for (int j = 0; j < 8; ++j) h[j] *= r;
       unpack8(pack8(h), h);  // h.to(bf16)
-      unpack8(w[c], wf);
+      unpack8(wv[k], wf);
 #pragma unroll
       for (int j = 0; j < 8; ++j) h[j] = wf[j] * h[j];
       out[c] = pack8(h);
@@ -95,24 +109,67 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const NormParams 
   }
 }
 
-// out = bf16(bf16(silu(gate)) * up), silu(g) = g / (1 + exp(-g)) in fp32 as torch's kernel
-// evaluates it; one thread per 8 elements.
+// out = bf16(bf16(silu(gate)) * up), silu(g) = g / (1 + e^-g) in fp32 (v_exp_f32 and v_rcp_f32; the bf16
+// result is that of torch's correctly rounded expf and division for all 65,536 gate values); grid
+// (column groups, rows), kSiluChunks chunks of 8 elements per thread, all of them loaded first.
+constexpr int kSiluChunks = 2;
+
+__device__ inline float silu(float g) {
+  if (g < -80.f) return g / (1.f + expf(-g));  // (1 / (1 + e^-g) is near or below the normal range)
+  // e^x = 2^hi (1 + lo ln 2), hi + lo = x log2(e): the rounding of the product x log2(e) alone would reach
+  // 2^-18 of e^x; the reciprocal takes one Newton step (both arguments finite: x >= -80)
+  const float x = -fminf(g, 80.f);
+  const float hi = x * kLog2e, lo = __builtin_fmaf(x, kLog2e, -hi);
+  const float e = fast_exp2(hi);
+  const float d = 1.f + __builtin_fmaf(e, lo * kLn2, e);
+  const float r = __builtin_amdgcn_rcpf(d);
+  return g * __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+}
+
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* gate, int64_t g_stride, const uint16_t* up,
                                                        int64_t u_stride, uint16_t* out, int64_t o_stride, int32_t rows,
                                                        int32_t width) {
   const int chunks = width >> 3;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= static_cast<int64_t>(rows) * chunks) return;
-  const int row = static_cast<int>(i / chunks), c = static_cast<int>(i - static_cast<int64_t>(row) * chunks);
-  float g[8], u[8];
-  unpack8(reinterpret_cast<const uint4*>(gate + row * g_stride)[c], g);
-  unpack8(reinterpret_cast<const uint4*>(up + row * u_stride)[c], u);
+  const int c0 = blockIdx.x * (256 * kSiluChunks) + threadIdx.x;
+  for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
+    const uint4* gr = reinterpret_cast<const uint4*>(gate + row * g_stride);
+    const uint4* ur = reinterpret_cast<const uint4*>(up + row * u_stride);
+    uint4* orow = reinterpret_cast<uint4*>(out + row * o_stride);
+    uint4 gv[kSiluChunks], uv[kSiluChunks];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) g[j] = g[j] / (1.f + expf(-g[j]));
-  unpack8(pack8(g), g);  // silu's bf16 result
+    for (int k = 0; k < kSiluChunks; ++k) {
+      const int c = min(c0 + 256 * k, chunks - 1);
+      gv[k] = load_nt(gr + c);
+      uv[k] = load_nt(ur + c);
+    }
 #pragma unroll
-  for (int j = 0; j < 8; ++j) g[j] *= u[j];
-  reinterpret_cast<uint4*>(out + row * o_stride)[c] = pack8(g);
+    for (int k = 0; k < kSiluChunks; ++k) {
+      if (c0 + 256 * k >= chunks) break;
+      float g[8], u[8];
+      unpack8(gv[k], g);
+      unpack8(uv[k], u);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) g[j] = silu(g[j]);
+      unpack8(pack8(g), g);  // silu's bf16 result
+#pragma unroll
+      for (int j = 0; j < 8; ++j) g[j] *= u[j];
+      orow[c0 + 256 * k] = pack8(g);
+    }
+  }
+}
+
+// The RMSNorm instance that holds a row of `hidden` elements.
+template <bool kAdd>
+void launch_rmsnorm(const NormParams& p, int32_t rows, hipStream_t s) {
+  const int chunks = (p.hidden + kNormThreads * 8 - 1) / (kNormThreads * 8);
+  if (chunks <= 1)
+    rmsnorm_kernel<kAdd, 1><<<rows, kNormThreads, 0, s>>>(p);
+  else if (chunks <= 2)
+    rmsnorm_kernel<kAdd, 2><<<rows, kNormThreads, 0, s>>>(p);
+  else if (chunks <= 4)
+    rmsnorm_kernel<kAdd, 4><<<rows, kNormThreads, 0, s>>>(p);
+  else
+    rmsnorm_kernel<kAdd, kNormMaxChunks><<<rows, kNormThreads, 0, s>>>(p);
 }
 
 }  // namespace
@@ -145,9 +202,9 @@ extern "C" int32_t lkv_rmsnorm(const lkv_rmsnorm_args* a, lkv_stream_t stream) {
   p.eps = a->eps;
   hipStream_t s = as_stream(stream);
   if (a->residual != nullptr)
-    rmsnorm_kernel<true><<<a->rows, kNormThreads, 0, s>>>(p);
+    launch_rmsnorm<true>(p, a->rows, s);
   else
-    rmsnorm_kernel<false><<<a->rows, kNormThreads, 0, s>>>(p);
+    launch_rmsnorm<false>(p, a->rows, s);
   return check_launch("lkv_rmsnorm");
 }
 
@@ -159,10 +216,11 @@ extern "C" int32_t lkv_silu_mul(const void* gate, int64_t gate_stride, const voi
   const uintptr_t align = reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) | reinterpret_cast<uintptr_t>(out);
   LKV_REQUIRE((align & 15) == 0, "rows must be 16-byte aligned");
   LKV_REQUIRE((gate_stride | up_stride | out_stride) % 8 == 0, "row strides must be multiples of 8 elements");
-  const int64_t threads = static_cast<int64_t>(rows) * (width / 8);
-  LKV_REQUIRE(threads / 256 < (1LL << 31), "too many elements");
-  if (threads == 0) return LKV_OK;
-  silu_mul_kernel<<<static_cast<unsigned>((threads + 255) / 256), 256, 0, as_stream(stream)>>>(
+  if (rows == 0) return LKV_OK;
+  constexpr int kPerBlock = 256 * 8 * kSiluChunks;
+  const dim3 grid(static_cast<unsigned>((static_cast<int64_t>(width) + kPerBlock - 1) / kPerBlock),
+                  static_cast<unsigned>(std::min(rows, 65535)));
+  silu_mul_kernel<<<grid, 256, 0, as_stream(stream)>>>(
       static_cast<const uint16_t*>(gate), gate_stride, static_cast<const uint16_t*>(up), up_stride,
       static_cast<uint16_t*>(out), out_stride, rows, width);
   return check_launch("lkv_silu_mul");
