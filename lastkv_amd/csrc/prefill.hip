@@ -26,6 +26,7 @@
 
 #include "attn_common.h"
 #include "common.h"
+#include "decode_body.h"
 #include "runtime.h"
 
 namespace lkv {
@@ -834,14 +835,13 @@ __device__ inline bool ragged_tile(const PrefillParams& p, int gt, int rows_per_
 // scan of cu_seqlens: a grid sized by the longest sequence for every sequence mostly exits, and the
 // exits delayed the working tiles (a serving step of 31 decode rows, a 1024-token row and a 7-token
 // row: 258 us for the one long row against 206 us for the same tiles alone).
-template <int NW, int CG, int WPE, bool kPaged>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) void prefill_kernel(
-    const PrefillParams p) {
-  __shared__ uint4 lds[kTileRing * kTileBuf];
+template <int NW, int CG, bool kPaged>
+__device__ __attribute__((always_inline)) inline void prefill_workgroup(const PrefillParams& p, const int wg, const int wgs,
+                                                                        uint4* lds) {
   // key splits: the grid is tile_splits copies of the tile grid, the split the slowest index
-  const int per_split = static_cast<int>(gridDim.x) / p.tile_splits;
-  const int split = static_cast<int>(blockIdx.x) / per_split;
-  const int id = static_cast<int>(blockIdx.x) - split * per_split;
+  const int per_split = wgs / p.tile_splits;
+  const int split = wg / per_split;
+  const int id = wg - split * per_split;
   int b, kvh, tile, tiles;
   if (p.cu != nullptr) {
     kvh = id % p.hkv;
@@ -858,6 +858,53 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) 
   prefill_tile<NW, CG, kPaged>(p, __builtin_amdgcn_readfirstlane(b), __builtin_amdgcn_readfirstlane(kvh),
                                __builtin_amdgcn_readfirstlane(p.causal ? tiles - 1 - tile : tile),
                                __builtin_amdgcn_readfirstlane(split), lds);
+}
+
+template <int NW, int CG, int WPE, bool kPaged>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) void prefill_kernel(
+    const PrefillParams p) {
+  __shared__ uint4 lds[kTileRing * kTileBuf];
+  prefill_workgroup<NW, CG, kPaged>(p, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), lds);
+}
+
+// A mixed serving step's decode rows (the decode kernel's 1-16 column class) and prefill tiles in one
+// launch: the decode rows are bound by HBM, the tiles by the matrix pipe and the VALU, and one launch after
+// the other each left the other's resource idle.  The decode items and as many tiles alternate in runs of
+// kMixRun workgroups (the dispatcher deals workgroups to the XCDs, their shader engines and CUs in turn, so
+// half of every engine's CUs take decode items, two each, and the other half tiles); the remaining tiles
+// follow and take the CUs of the decode items that end.  31 decode rows at 8K, a 1024-token row and a
+// 7-token row: the step 374 -> 325 us; runs of 32 to 128 alike, runs of 256 (a decode item beside a tile on
+// every CU) 366, of 8 (whole shader engines of one kind) 395, decode items first 367.
+constexpr int kMixRun = 64;
+
+// Workgroups of a mixed launch with `dec` decode items and `tiles` tile workgroups (both interleaved up to
+// the next multiple of kMixRun).
+inline int64_t mixed_grid(int64_t dec, int64_t tiles) {
+  const int64_t runs = (dec + kMixRun - 1) / kMixRun * kMixRun;
+  return runs + std::max(tiles, runs);
+}
+
+template <bool kPaged, bool kVScale, bool kNT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void mixed_step_kernel(
+    const PrefillParams p, const DecodeParams d, const int dec_wgs, const int tile_wgs) {
+  __shared__ uint4 lds[kTileRing * kTileBuf];
+  static_assert(sizeof(DecodeShared<1>) <= sizeof(lds), "the decode rows' states fit the tiles' LDS");
+  const int runs = (dec_wgs + kMixRun - 1) / kMixRun * kMixRun;
+  int wg = static_cast<int>(blockIdx.x) - runs;
+  bool dec = false;
+  if (wg < runs) {  // the alternating part
+    const int run = static_cast<int>(blockIdx.x) / kMixRun;
+    dec = (run & 1) == 0;
+    wg = (run >> 1) * kMixRun + static_cast<int>(blockIdx.x) % kMixRun;
+  }
+  if (dec) {
+    DecodeItem it;
+    if (wg >= dec_wgs || !decode_item<true>(d, wg, it)) return;  // (workgroup-uniform)
+    decode_split_body<kVScale, kNT, true, 1, false, false>(d, it, *reinterpret_cast<DecodeShared<1>*>(lds));
+    return;
+  }
+  if (wg >= tile_wgs) return;
+  prefill_workgroup<4, 2, kPaged>(p, wg, tile_wgs, lds);
 }
 
 // Merges the key splits of one (row, query head) per wave: O = sum_s 2^(lse_s - lse) O_s with
@@ -1159,6 +1206,24 @@ void launch_tiles(int waves, bool paged, dim3 grid, const lkv::PrefillParams& p,
     prefill_kernel<2, 2, 1, false><<<grid, 2 * 64, 0, s>>>(p);
 }
 
+// The class's decode work items and the tiles of a ragged call in one launch.
+void launch_mixed(bool paged, int64_t tile_wgs, const lkv::PrefillParams& p, const lkv::ShortRowsPlan& d, hipStream_t s) {
+  using namespace lkv;
+  const int dec = static_cast<int>(d.items);
+  const dim3 grid(static_cast<unsigned>(mixed_grid(dec, tile_wgs)));
+  const int which = (paged ? 4 : 0) + (d.vscale ? 2 : 0) + (d.nt ? 1 : 0);
+  switch (which) {
+    case 0: mixed_step_kernel<false, false, false><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+    case 1: mixed_step_kernel<false, false, true><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+    case 2: mixed_step_kernel<false, true, false><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+    case 3: mixed_step_kernel<false, true, true><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+    case 4: mixed_step_kernel<true, false, false><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+    case 5: mixed_step_kernel<true, false, true><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+    case 6: mixed_step_kernel<true, true, false><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+    default: mixed_step_kernel<true, true, true><<<grid, 256, 0, s>>>(p, d.p, dec, static_cast<int>(tile_wgs)); break;
+  }
+}
+
 // The wide-range V instance for the same wave count and addressing, over `pair_wgs` workgroups
 // (4-wave tiles at one wave per SIMD: the bf16 instance needs more than 256 registers).
 void launch_wide(int waves, bool paged, int pair_wgs, const lkv::PrefillParams& p, hipStream_t s) {
@@ -1233,11 +1298,35 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
   // kernel, also with tile_waves 4 or 8 unless all of its sequences are short.
   const int64_t max_cols = seq_tokens * group;
   const bool short_on_decode = a->tile_waves == 0 || ragged_short_on_decode(a);
+  const TilePlan plan = tile_plan(a);
+  // key splits: as many as the workspace holds the states of (1 without room)
+  int splits = plan.splits;
+  const int64_t v16_bytes = v16_region_bytes(a, vblocks);
+  while (splits > 1 && v16_bytes + tile_split_bytes(a, plan, splits) > a->workspace_bytes) --splits;
+  if (vblocks == 0) splits = 1;
+  ShortRowsPlan rows16;  // the 1-16 column class, when it runs in one launch with the tiles
+  bool mixed = false;
   if (short_on_decode) {
     // (with the host copy of a ragged call's offsets: only the classes that hold a sequence)
     const HostPlan hp = host_plan(a, group);
     const int32_t bounds[4] = {0, 16, 32, 64};
+    // A step whose class of 1-16 columns and whose tiles both hold sequences runs the two in one launch
+    // (mixed_step_kernel), when the host knows the class's count (its grid then holds exactly its work
+    // items), the split counts are the library's and the class's split states fit behind the tiles' (in
+    // the launch of their own they are the workspace's first bytes, which the pre-pass writes here).
+    if (hp.known && hp.any_tile && hp.class_n[0] > 0 && plan.waves == 4 && a->num_splits == 0 && vblocks > 0) {
+      const int64_t used = (v16_bytes + tile_split_bytes(a, plan, splits) + 15) / 16 * 16;
+      if (const int32_t st = plan_short_rows(a, p.seg, group, 0, 16, hp.class_n[0], nullptr, int64_t{1} << 62, rows16)) return st;
+      const int64_t room = std::max<int64_t>(0, a->workspace_bytes - used);
+      mixed = !rows16.empty && (rows16.p.splits == 1 || rows16.state_bytes <= room);
+      if (mixed && rows16.p.splits > 1) {
+        if (const int32_t st = plan_short_rows(a, p.seg, group, 0, 16, hp.class_n[0],
+                                               static_cast<uint8_t*>(a->workspace) + used, room, rows16))
+          return st;
+      }
+    }
     for (int c = 0; c < 3; ++c) {
+      if (c == 0 && mixed) continue;
       if (max_cols <= bounds[c]) break;
       // a uniform call is one class: the one its width falls in
       if (!ragged && max_cols > bounds[c + 1]) continue;
@@ -1272,15 +1361,9 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
   p.rows = a->tokens;
   p.decode_rows = ragged && short_on_decode ? 64 : -1;
   const int64_t heads = static_cast<int64_t>(a->num_kv_heads) * a->batch;
-  const TilePlan plan = tile_plan(a);
   const int waves = plan.waves;
   const int64_t tiles = plan.tiles, wgs = plan.wgs;
-  // key splits: as many as the workspace holds the states of (1 without room)
-  int splits = plan.splits;
-  const int64_t v16_bytes = v16_region_bytes(a, vblocks);
-  while (splits > 1 && v16_bytes + tile_split_bytes(a, plan, splits) > a->workspace_bytes) --splits;
-  if (vblocks == 0) splits = 1;
-  LKV_REQUIRE(wgs * splits < (1LL << 31), "too many query rows");
+  LKV_REQUIRE((mixed ? mixed_grid(rows16.items, wgs * splits) : wgs * splits) < (1LL << 31), "too many query rows");
   p.tile_splits = splits;
   p.ws_o = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(a->workspace) + v16_bytes) : nullptr;
   p.ws_lse = splits > 1 ? p.ws_o + plan.rows_all * a->num_q_heads * splits * kHeadDim : nullptr;
@@ -1302,9 +1385,14 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
       v16_stage_kernel<false, 1><<<vgrid, 256, 0, s>>>(p);
     if (const int32_t e = check_launch("lkv_prefill_attn (V pre-pass)")) return e;
   }
-  const dim3 grid(static_cast<unsigned>(wgs * splits));
-  launch_tiles(waves, paged, grid, p, s);
-  if (const int32_t e = check_launch("lkv_prefill_attn")) return e;
+  if (mixed) {
+    launch_mixed(paged, wgs * splits, p, rows16, s);
+    if (const int32_t e = check_launch("lkv_prefill_attn (decode rows and tiles)")) return e;
+    if (const int32_t e = combine_short_rows(rows16, s, "lkv_prefill_attn (decode rows' merge)")) return e;
+  } else {
+    launch_tiles(waves, paged, dim3(static_cast<unsigned>(wgs * splits)), p, s);
+    if (const int32_t e = check_launch("lkv_prefill_attn")) return e;
+  }
   if (vblocks == 0) return LKV_OK;
   // the tiles that read a V value of magnitude 65536 or more (flagged by the pre-pass; the instance
   // above skipped them), exactly in bf16, by workgroups that each scan one (sequence, kv head)'s

@@ -231,6 +231,39 @@ def test_ragged_host_offsets_plan_the_same_results(case):
                               cu_seqlens_q_host=cu[:-1], **seg)
 
 
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("decode_rows,tile_rows", [(1, [17]), (9, [33, 70]), (70, [100]), (150, [400, 20])])
+def test_ragged_decode_rows_beside_tiles_in_one_launch(decode_rows, tile_rows, paged):
+    """With the host copy of the offsets a step's decode rows and tiles run in one launch (decode items and
+    tiles interleaved in runs of 64 workgroups): 1 to 150 rows, so fewer and more items than one run, with
+    32 splits to one, more and fewer tiles than decode items.  Outputs and LSE equal the separate launches
+    (no host copy) bit for bit, with room for the rows' split states behind the tiles' and without."""
+
+    rng = np.random.default_rng(900 + decode_rows)
+    lengths = [1] * (decode_rows // 2) + tile_rows + [1] * (decode_rows - decode_rows // 2)
+    Hkv, G = 2, 4
+    Hq = Hkv * G
+    seg, ks, vs, _ = _ragged_case(rng, lengths, Hkv, G, paged, True)
+    cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    T = int(cu[-1])
+    q = _bf(rng, (T, Hq, 128))
+    cu_t = torch.from_numpy(cu).to(DEV)
+    kw = dict(causal=True, cu_seqlens_q=cu_t, max_seqlen_q=max(lengths))
+    roomy = torch.empty(256 << 20, dtype=torch.uint8, device=DEV)
+    results = []
+    for host, ws in ((None, None), (cu, None), (cu, roomy)):
+        lse = torch.full((T, Hq), 7.0, dtype=torch.float32, device=DEV)
+        results.append((ops.prefill_attention(_t(q), lse=lse, cu_seqlens_q_host=host, workspace=ws, **kw, **seg), lse))
+    for out, lse in results[1:]:
+        assert torch.equal(out, results[0][0]) and torch.equal(lse, results[0][1])
+    for b in (0, decode_rows // 2, len(lengths) - 1):
+        rows = slice(int(cu[b]), int(cu[b + 1]))
+        want, _ = A.attention(q[rows].transpose(1, 0, 2)[None], ks[b], vs[b], causal_bottom_right=True)
+        want = bf16.round_bf16(want[0].transpose(1, 0, 2).astype(np.float32))
+        got = results[2][0][rows].float().cpu().numpy()
+        assert A.max_abs(got, want) <= MAX_ABS and A.rel_l2(got, want) <= REL_L2, (lengths, b)
+
+
 RAGGED_SWEEP_SEED0 = 7000
 RAGGED_SWEEP_CASES = 60
 RAGGED_SWEEP_PART = 10
