@@ -1,7 +1,8 @@
-"""Compile the gfx950 HIP sources of this package into ``lastkv_amd/liblastkv_amd.so``.
+"""Compile the native code of this package: ``liblastkv_amd.so`` and the extension module ``_host.so``.
 
 Every ``csrc/*.hip`` file is compiled with hipcc for gfx950 only, then linked into one shared
-library exporting the C ABI declared in ``include/lastkv_amd.h``.  Run as
+library exporting the C ABI declared in ``include/lastkv_amd.h``.  ``csrc/host.cpp`` (host code
+only) becomes the module ``lastkv_amd._host`` against the installed torch.  Run as
 ``python -m lastkv_amd.build``.
 """
 
@@ -13,12 +14,14 @@ import pathlib
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = pathlib.Path(__file__).resolve().parent
 REPO_DIR = PKG_DIR.parent
 CSRC = PKG_DIR / "csrc"
 LIB_NAME = "liblastkv_amd.so"
 LIB_PATH = PKG_DIR / LIB_NAME
+HOST_PATH = PKG_DIR / "_host.so"
 OBJ_DIR = PKG_DIR / "_build"
 
 ARCH = "gfx950"
@@ -55,15 +58,34 @@ def _compile(src: pathlib.Path, verbose: bool) -> pathlib.Path:
     return obj
 
 
+def _build_host() -> None:
+    import torch
+
+    root = pathlib.Path(torch.__file__).resolve().parent
+    includes = [root / "include", root / "include/torch/csrc/api/include", sysconfig.get_paths()["include"],
+                pathlib.Path(_hipcc()).resolve().parents[1] / "include"]
+    tmp = HOST_PATH.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(x for i in includes for x in ("-isystem", str(i))), str(CSRC / "host.cpp"), "-o", str(tmp),
+           f"-L{root / 'lib'}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"compiling host.cpp failed:\n{proc.stdout}{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose: bool = False) -> pathlib.Path:
-    """Compile every HIP source and link ``liblastkv_amd.so``; returns its path."""
+    """Compile every HIP source and link ``liblastkv_amd.so``, and build ``_host.so``; returns the library's path."""
 
     OBJ_DIR.mkdir(exist_ok=True)
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
         raise RuntimeError(f"no HIP sources under {CSRC}")
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources))) as pool:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources) + 1)) as pool:
+        host = pool.submit(_build_host)
         objs = list(pool.map(lambda s: _compile(s, verbose), sources))
+        host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     proc = subprocess.run(cmd, capture_output=True, text=True)

@@ -3,6 +3,10 @@
 Each wrapper validates shapes, dtypes and devices, then passes raw device pointers and the
 current HIP stream of the tensors' device to ``liblastkv_amd.so``.  Nothing here computes on
 the CPU; a missing library raises ``LastKVNativeError``.
+
+The hot ops (attention, epilogue, RMSNorm, SwiGLU) first hand their arguments to ``_host``
+(csrc/host.cpp), which makes the same checks and the same call natively for the common argument
+forms; where it answers None, the Python body below it checks, reports and calls as it always did.
 """
 
 from __future__ import annotations
@@ -15,6 +19,11 @@ import numpy as np
 import torch
 
 from . import _lib
+
+try:
+    from . import _host
+except ImportError:  # not built: _bind_host raises at the first call
+    _host = None
 
 HEAD_DIM = 128
 BLOCK_TOKENS = 32
@@ -150,6 +159,27 @@ class PagedKV:
         return self.k.device
 
 
+_host_bound = False
+
+
+def _bind_host() -> bool:
+    """Give ``_host`` the library's entry points (once per process); False when the library is missing
+    (the Python bodies then raise after their own checks)."""
+
+    global _host_bound
+    try:
+        lib = _lib.load()
+    except _lib.LastKVNativeError:
+        return False
+    if _host is None:
+        raise _lib.LastKVNativeError("_host.so is not built; run `python -m lastkv_amd.build`")
+    names = ("lkv_decode_attn", "lkv_decode_workspace_bytes", "lkv_prefill_attn", "lkv_prefill_workspace_bytes",
+             "lkv_qkv_epilogue", "lkv_rmsnorm", "lkv_silu_mul")
+    _host.bind(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), TiledKV, PagedKV)
+    _host_bound = True
+    return True
+
+
 def cache_pack(src: torch.Tensor, cache: torch.Tensor, kind: int, token0: int = 0, *, capacity_tokens: int | None = None) -> None:
     """Write ``src`` ``[B, H, T, 128]`` into cache tokens ``[token0, token0 + T)`` of slots ``0..B-1``."""
 
@@ -205,6 +235,8 @@ def _cu_count(device: torch.device) -> int:
     index = device.index if device.index is not None else torch.cuda.current_device()
     if index not in _CU_COUNT:
         _CU_COUNT[index] = int(torch.cuda.get_device_properties(index).multi_processor_count)
+        if _host is not None:
+            _host.set_cu_count(index, _CU_COUNT[index])
     return _CU_COUNT[index]
 
 
@@ -350,6 +382,12 @@ def decode_attention(
     nothing); calls overlapping on one GPU then race.
     """
 
+    if not no_alloc and (_host_bound or _bind_host()):
+        done = _host.decode_attention(q, older, older_len, older_slot, vscale, local, local_len, local_start, local_slot,
+                                      older_table, local_table, local_ring_blocks, sm_scale, num_splits, out, lse, workspace,
+                                      kv_cache_hint, out_scale)
+        if done is not None:
+            return done
     _require_bf16_cuda("q", q)
     if q.dim() == 4:
         _require(q.shape[2] == 1, "decode_attention takes one query token per sequence")
@@ -453,6 +491,12 @@ def prefill_attention(
     head, and its shorter ones stay on the decode kernel unless all of its sequences are short.
     ``out_scale`` as in ``decode_attention``."""
 
+    if _host_bound or _bind_host():
+        done = _host.prefill_attention(q, older, older_len, older_slot, vscale, local, local_len, local_start, local_slot,
+                                       older_table, local_table, local_ring_blocks, causal, sm_scale, out, lse, workspace,
+                                       tile_waves, out_scale, cu_seqlens_q, max_seqlen_q, num_splits, cu_seqlens_q_host)
+        if done is not None:
+            return done
     _require_bf16_cuda("q", q)
     ragged = cu_seqlens_q is not None
     if ragged:
@@ -697,6 +741,12 @@ def qkv_epilogue(
     writes the ring's V as ``bf16(v * ring_v_mul[g])`` (the vLLM path's V / s rings); the shared
     cache keeps the raw V."""
 
+    if _host_bound or _bind_host():
+        done = _host.qkv_epilogue(q, k, v, cos, sin, num_q_heads, num_kv_heads, q_norm_weight, k_norm_weight, eps, positions,
+                                  ring, ring_slot, deep, deep_slot, q_out, ring_table, ring_tokens, deep_table,
+                                  ROUNDINGS.get(rounding), ring_v_mul, cu_seqlens, max_seqlen)
+        if done is not None:
+            return done
     ragged = cu_seqlens is not None
     if ragged:
         _require(cu_seqlens.dtype == torch.int32 and cu_seqlens.dim() == 1 and cu_seqlens.numel() >= 2
@@ -910,6 +960,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, *, residual: torc
     """LlamaRMSNorm of the rows of ``x`` (bf16 ``[..., hidden]``); with ``residual`` first
     ``residual += x`` in bf16 (in place) and the sum is normalised.  Returns ``out``."""
 
+    if _host_bound or _bind_host():
+        done = _host.rmsnorm(x, weight, eps, residual, out)
+        if done is not None:
+            return done
     rows, hidden, xs = _rows2d("x", x)
     _require_bf16_cuda("weight", weight)
     _require(weight.is_contiguous() and weight.numel() == hidden, "weight must be a contiguous bf16 [hidden] tensor")
@@ -935,6 +989,10 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float, *, residual: torc
 def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     """``F.silu(gate) * up`` for bf16 ``[..., width]`` tensors, as torch rounds it."""
 
+    if _host_bound or _bind_host():
+        done = _host.silu_mul(gate, up, out)
+        if done is not None:
+            return done
     rows, width, gs = _rows2d("gate", gate)
     u_rows, u_width, us = _rows2d("up", up)
     _require((u_rows, u_width) == (rows, width), "up shape must match gate")
