@@ -448,7 +448,9 @@ constexpr int kTileBuf = 1024;     // uint4 per block buffer (16 KiB)
 // kWide: the instance for tiles whose V does not fit fp16 (the pre-pass flagged one of their blocks):
 // V staged as bf16 from the caches (older blocks as bf16(V * s)), P split into bf16 hi + lo, P V and
 // the row sums on bf16 MFMAs; the fp16 instance skips those tiles and this one runs only them.
-template <int NW, int CG, bool kPaged, bool kWide = false>
+// KS = 2: the workgroup has NW waves for each half of the split's keys (2 NW in all, both on the same
+// query rows, each half with an LDS ring of its own); the halves' states are merged through LDS at the end.
+template <int NW, int CG, bool kPaged, bool kWide = false, int KS = 1>
 __device__ __attribute__((always_inline)) inline void prefill_tile(const PrefillParams& p, const int b, const int kvh,
                                                                    const int tile, const int split, uint4* lds) {
   constexpr bool kSplitP = NW == 2 || kWide;
@@ -460,7 +462,10 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
   constexpr int kRowsPerWg = NW * kRowsPerWave;
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = KS == 1 ? 0 : wave_all / NW;
+  const int wave = wave_all - half * NW;
+  uint4* const ring = lds + half * (kTileRing * kTileBuf);
   const int n16 = lane & 15, g4 = lane >> 4;
   const int G = p.group;
   const SeqRows sr = seq_rows(p, b);
@@ -490,24 +495,38 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
     if (!needs_wide) return;
   }
   const float vs_older = p.vscale_mode ? p.vscale[kvh] : 1.f;  // (the wide instance's V scale)
-  // this split's blocks [kb0, kb1) (the wide instance runs every block as split 0)
-  const int S = kWide ? 1 : p.tile_splits;
+  // this split's blocks [kb0, kb1) (the wide instance runs every block as split 0); with KS = 2 key
+  // split s is halves 2 s and 2 s + 1 of twice as many splits
+  const int S = kWide ? 1 : p.tile_splits * KS;
   int kb0 = 0, kb1 = nbt;
+  int steps = 0;  // the blocks of the longer half (both halves pass as many barriers)
   if (S > 1) {
     // as many equal splits as start inside the older segment (a short older segment would leave
     // the last split most of the keys: slower than no split)
     int se = min(S, sv.nb0);
     while (se > 1 && (se - 1) * ((nbt + se - 1) / se) > sv.nb0 - 1) --se;
-    if (split >= max(se, 1)) {
-      kb1 = 0;
-    } else if (se > 1) {
-      const int q = (nbt + se - 1) / se;
-      kb0 = split * q;
-      if (split + 1 < se) kb1 = (split + 1) * q;
+    const int q = (nbt + max(se, 1) - 1) / max(se, 1);
+    auto range = [&](int s) {
+      int2 r = make_int2(0, nbt);
+      if (s >= max(se, 1)) {
+        r.y = 0;
+      } else if (se > 1) {
+        r.x = s * q;
+        if (s + 1 < se) r.y = (s + 1) * q;
+      }
+      return r;
+    };
+    const int2 mine = range(split * KS + half);
+    kb0 = mine.x;
+    kb1 = mine.y;
+    if (KS == 2) {
+      const int2 other = range(split * KS + 1 - half);
+      steps = max(max(kb1 - kb0, other.y - other.x), 0);
     }
   }
   kb0 = __builtin_amdgcn_readfirstlane(kb0);
   kb1 = __builtin_amdgcn_readfirstlane(kb1);
+  steps = __builtin_amdgcn_readfirstlane(steps);
 
   uint4 qf[CG][4];
   int lim[CG];  // last visible local-segment token of this lane's column
@@ -565,7 +584,7 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
                             min(kb0 + j, last), wave, lane_off);
 #pragma unroll
     for (int j = 0; j < kDist; ++j) {
-      stage_store<NW, kWide>(sets[j % kStages], lds + j * kBuf, wave, lane, vs_of(min(kb0 + j, last)));
+      stage_store<NW, kWide>(sets[j % kStages], ring + j * kBuf, wave, lane, vs_of(min(kb0 + j, last)));
       const int lb = min(kb0 + j + kStages, last);
       stage_load<NW, kWide>(sets[j % kStages], rsrc, k_block<kPaged>(sv, lb), vb(lb), lb, wave, lane_off);
     }
@@ -585,8 +604,8 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
       for (int u = 0; u < 2; ++u) sc[cg][u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
-      const uint4 k0 = lds[kb * 64 + lane];
-      const uint4 k1 = lds[(4 + kb) * 64 + lane];
+      const uint4 k0 = ring[kb * 64 + lane];
+      const uint4 k1 = ring[(4 + kb) * 64 + lane];
 #pragma unroll
       for (int cg = 0; cg < CG; ++cg) {
         sc[cg][0] = mfma_bf16(k0, qf[cg][kb], sc[cg][0]);
@@ -623,9 +642,9 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
     // blocks per wave at the causal edge).
     auto step = [&](auto rc, int blk) __attribute__((always_inline)) {
       constexpr int R = decltype(rc)::value;
-      const uint4* cur = lds + R * kBuf;
-      const uint4* nxt = lds + ((R + 1) % kRing) * kBuf;
-      uint4* wr = lds + ((R + kDist) % kRing) * kBuf;
+      const uint4* cur = ring + R * kBuf;
+      const uint4* nxt = ring + ((R + 1) % kRing) * kBuf;
+      uint4* wr = ring + ((R + kDist) % kRing) * kBuf;
       // the register set holding block i + kDist (loaded kStages steps ago)
       Stage<NW>& st = sets[(R + kDist) % kStages];
       const int ld_blk = min(blk + kDist + kStages, last);
@@ -755,6 +774,40 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
       if (blk + decltype(jc)::value < kb1) step(jc, blk + decltype(jc)::value);
     });
   }
+  if constexpr (KS == 2) {
+    if (kb1 <= kb0) {  // an empty half: the other's wide test and prologue barrier
+      if (flags_any(flag_peek, p, b, kvh, nbt)) return;
+      if (steps > 0) __syncthreads();
+    }
+    for (int i = max(kb1 - kb0, 0); i < steps; ++i) __syncthreads();
+    // Merge: the second half leaves O in its own ring (64 KiB, in lane order) and its offsets and row sums
+    // in the first's (every wave has passed the last step's barrier, so no ring is read any more); the
+    // first half takes O = O0 2^(mc0 - mc) + O1 2^(mc1 - mc), mc the larger offset of a non-empty half.
+    static_assert(NW * CG * 8 * 64 <= kTileRing * kTileBuf, "the second half's O fits its ring");
+    f32x4* const so = reinterpret_cast<f32x4*>(lds + kTileRing * kTileBuf) + wave * (CG * 8 * 64) + lane;
+    float2* const sl = reinterpret_cast<float2*>(lds) + wave * (CG * 64) + lane;
+    if (half == 1) {
+#pragma unroll
+      for (int cg = 0; cg < CG; ++cg) {
+        sl[cg * 64] = make_float2(rs[cg].mc, ol[cg][0]);
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb) so[(cg * 8 + nb) * 64] = o[cg][nb];
+      }
+    }
+    __syncthreads();
+    if (half == 1) return;
+#pragma unroll
+    for (int cg = 0; cg < CG; ++cg) {
+      const float2 other = sl[cg * 64];
+      const float m0 = ol[cg][0] > 0.f ? rs[cg].mc : kNegInf, m1 = other.y > 0.f ? other.x : kNegInf;
+      const float m = fmaxf(m0, m1);
+      const float w0 = m0 == kNegInf ? 0.f : fast_exp2(m0 - m), w1 = m1 == kNegInf ? 0.f : fast_exp2(m1 - m);
+      rs[cg].mc = m == kNegInf ? 0.f : m;
+      ol[cg][0] = ol[cg][0] * w0 + other.y * w1;
+#pragma unroll
+      for (int nb = 0; nb < 8; ++nb) o[cg][nb] = o[cg][nb] * w0 + so[(cg * 8 + nb) * 64] * w1;
+    }
+  }
 
   // normalise and write: lane (n16, g4) holds dims 16 * nb + 4 * g4 + i of row n16 of each group
   const float os = p.out_scale != nullptr ? p.out_scale[kvh] : 1.f;
@@ -835,7 +888,7 @@ __device__ inline bool ragged_tile(const PrefillParams& p, int gt, int rows_per_
 // scan of cu_seqlens: a grid sized by the longest sequence for every sequence mostly exits, and the
 // exits delayed the working tiles (a serving step of 31 decode rows, a 1024-token row and a 7-token
 // row: 258 us for the one long row against 206 us for the same tiles alone).
-template <int NW, int CG, bool kPaged>
+template <int NW, int CG, bool kPaged, int KS = 1>
 __device__ __attribute__((always_inline)) inline void prefill_workgroup(const PrefillParams& p, const int wg, const int wgs,
                                                                         uint4* lds) {
   // key splits: the grid is tile_splits copies of the tile grid, the split the slowest index
@@ -855,16 +908,16 @@ __device__ __attribute__((always_inline)) inline void prefill_workgroup(const Pr
     b = logical / (tiles * p.hkv);
   }
   // (one call site: the tile body is inlined once)
-  prefill_tile<NW, CG, kPaged>(p, __builtin_amdgcn_readfirstlane(b), __builtin_amdgcn_readfirstlane(kvh),
-                               __builtin_amdgcn_readfirstlane(p.causal ? tiles - 1 - tile : tile),
-                               __builtin_amdgcn_readfirstlane(split), lds);
+  prefill_tile<NW, CG, kPaged, false, KS>(p, __builtin_amdgcn_readfirstlane(b), __builtin_amdgcn_readfirstlane(kvh),
+                                          __builtin_amdgcn_readfirstlane(p.causal ? tiles - 1 - tile : tile),
+                                          __builtin_amdgcn_readfirstlane(split), lds);
 }
 
-template <int NW, int CG, int WPE, bool kPaged>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) void prefill_kernel(
+template <int NW, int CG, int WPE, bool kPaged, int KS = 1>
+__global__ __launch_bounds__(NW * KS * 64) __attribute__((amdgpu_waves_per_eu(WPE))) void prefill_kernel(
     const PrefillParams p) {
-  __shared__ uint4 lds[kTileRing * kTileBuf];
-  prefill_workgroup<NW, CG, kPaged>(p, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), lds);
+  __shared__ uint4 lds[KS * kTileRing * kTileBuf];
+  prefill_workgroup<NW, CG, kPaged, KS>(p, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), lds);
 }
 
 // A mixed serving step's decode rows (the decode kernel's 1-16 column class) and prefill tiles in one
@@ -1190,9 +1243,13 @@ extern "C" int64_t lkv_prefill_workspace_min_bytes(const lkv_prefill_args* a) {
 }
 
 // The tile kernel instance for this call's wave count and addressing.
-void launch_tiles(int waves, bool paged, dim3 grid, const lkv::PrefillParams& p, hipStream_t s) {
+void launch_tiles(int waves, bool halves, bool paged, dim3 grid, const lkv::PrefillParams& p, hipStream_t s) {
   using namespace lkv;
-  if (waves == 8 && paged)
+  if (halves && paged)
+    prefill_kernel<4, 2, 2, true, 2><<<grid, 8 * 64, 0, s>>>(p);
+  else if (halves)
+    prefill_kernel<4, 2, 2, false, 2><<<grid, 8 * 64, 0, s>>>(p);
+  else if (waves == 8 && paged)
     prefill_kernel<8, 2, 2, true><<<grid, 8 * 64, 0, s>>>(p);
   else if (waves == 8)
     prefill_kernel<8, 2, 2, false><<<grid, 8 * 64, 0, s>>>(p);
@@ -1364,6 +1421,18 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
   const int waves = plan.waves;
   const int64_t tiles = plan.tiles, wgs = plan.wgs;
   LKV_REQUIRE((mixed ? mixed_grid(rows16.items, wgs * splits) : wgs * splits) < (1LL << 31), "too many query rows");
+  // Pairs of 4-wave key splits share a workgroup of 8 waves and merge in LDS, when half as many workgroups
+  // still fill the CUs (at least 3/4 of the rounds they take): the states' round trip through memory and,
+  // for 2 splits, the merge launch go.  One sequence's 1024 tokens at 7K (256 tiles, 2 splits) 152.4 ->
+  // 140.3 us, 1000 at 3K 127.5 -> 116.0, 512 at 8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line 200
+  // tokens at 5K (56 tiles, 4 splits) would take 59.5 instead of 51.3 and two sequences' 300 at 3K (160
+  // tiles, 4 splits: 320 workgroups, a second round of 64) 81.6 instead of 78.0.  Uniform calls only: a
+  // ragged call's tiles keep one arithmetic whether or not they share a launch with decode rows.
+  const int64_t cu_count = device_cu_count() > 0 ? device_cu_count() : 256;
+  const int64_t half_wgs = wgs * splits / 2;
+  const bool halves = waves == 4 && splits % 2 == 0 && !ragged && half_wgs >= cu_count &&
+                      half_wgs * 4 >= (half_wgs + cu_count - 1) / cu_count * cu_count * 3;
+  if (halves) splits /= 2;
   p.tile_splits = splits;
   p.ws_o = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(a->workspace) + v16_bytes) : nullptr;
   p.ws_lse = splits > 1 ? p.ws_o + plan.rows_all * a->num_q_heads * splits * kHeadDim : nullptr;
@@ -1390,15 +1459,14 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
     if (const int32_t e = check_launch("lkv_prefill_attn (decode rows and tiles)")) return e;
     if (const int32_t e = combine_short_rows(rows16, s, "lkv_prefill_attn (decode rows' merge)")) return e;
   } else {
-    launch_tiles(waves, paged, dim3(static_cast<unsigned>(wgs * splits)), p, s);
+    launch_tiles(waves, halves, paged, dim3(static_cast<unsigned>(wgs * splits)), p, s);
     if (const int32_t e = check_launch("lkv_prefill_attn")) return e;
   }
   if (vblocks == 0) return LKV_OK;
   // the tiles that read a V value of magnitude 65536 or more (flagged by the pre-pass; the instance
   // above skipped them), exactly in bf16, by workgroups that each scan one (sequence, kv head)'s
   // flags at a time
-  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
-  launch_wide(waves, paged, static_cast<int>(std::min(heads, cus)), p, s);
+  launch_wide(waves, paged, static_cast<int>(std::min(heads, cu_count)), p, s);
   if (const int32_t e = check_launch("lkv_prefill_attn (wide-range V)")) return e;
   if (splits == 1) return LKV_OK;
   const int64_t items = plan.rows_all * a->num_q_heads;  // (row, query head) pairs, 4 per workgroup

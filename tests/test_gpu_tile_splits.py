@@ -113,3 +113,35 @@ def test_ragged_step_long_row_takes_key_splits():
         worst = max(worst, A.rel_l2(got, want))
         assert A.max_abs(got, want) <= MAX_ABS and A.rel_l2(got, want) <= REL_L2, f"sequence {b}"
     print(f"ragged step with a long row: worst rel_l2 {worst:.2e}", flush=True)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("T0,L,causal,wide", [(1500, 1024, True, False), (1500, 1024, False, False), (1501, 1021, True, False),
+                                              (33, 1024, True, False), (1500, 1024, True, True), (800, 513, True, False)])
+def test_key_halves_of_one_workgroup_match_oracle(T0, L, causal, wide, paged):
+    """Uniform calls whose pairs of key splits share a workgroup (256 tiles of 128 rows: two halves; 129 row
+    tiles x 2 kv heads with four splits: two halves of two splits): equal and unequal halves, a ragged last
+    block, an older segment too short to split (the second half is empty) and a V value fp16 cannot hold
+    (whose tiles run on the wide instance)."""
+
+    rng = np.random.default_rng(31 + T0 + L + causal + 2 * paged)
+    B, Hkv, G = 1, 2, 16
+    seg, k, v = _case(rng, B, Hkv, T0, L, paged)
+    if wide:
+        seg["vscale"] = seg["vscale"] * 2.0 ** 17
+        v = v.copy()
+        v[:, :, :T0] *= 2.0 ** 17  # (a power of two: bf16(V s 2^17) = 2^17 bf16(V s))
+    q = _bf(rng, (B, L, Hkv * G, 128))
+    lse = torch.empty((B, L, Hkv * G), dtype=torch.float32, device=DEV)
+    got = ops.prefill_attention(_t(q), causal=causal, lse=lse, **seg).float()
+    kt, vt, qt = (torch.from_numpy(np.ascontiguousarray(x)).to(DEV).double() for x in (k[0], v[0], q[0]))
+    n = kt.shape[1]
+    hide = torch.arange(n, device=DEV)[None, :] > (n - L + torch.arange(L, device=DEV))[:, None]
+    for h in range(0, Hkv * G, 5):
+        s = qt[:, h] @ kt[h // G].t().contiguous() / 128 ** 0.5
+        if causal:
+            s = s.masked_fill(hide, float("-inf"))
+        want = torch.softmax(s, -1) @ vt[h // G]
+        torch.testing.assert_close(lse[0, :, h].double(), torch.logsumexp(s, -1), rtol=1e-4, atol=1e-4)
+        want = want.bfloat16().double()
+        assert float((got[0, :, h].double() - want).norm() / want.norm()) <= REL_L2
