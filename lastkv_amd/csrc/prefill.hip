@@ -432,6 +432,23 @@ constexpr int kMaxTileSplits = 4;  // key splits of a tile (the wide instance ma
 constexpr int kTileRing = 4;       // LDS block buffers of the tile kernel
 constexpr int kTileBuf = 1024;     // uint4 per block buffer (16 KiB)
 
+// The key splits a tile of nbt key blocks, nb0 of them older ones, takes of S offered: 4-wave tiles as many
+// as leave each kMinSplitBlocks, wherever they start (a row that sees no key in its split's first block
+// takes its reference from the first block it sees).  Wider tiles, whose loop does not test for such rows,
+// and calls with an older segment of 1 to kMinOlderBlocks - 1 blocks (no chunk of 256 tokens or more leaves
+// one so short): as many equal ones as start inside the older segment, whose blocks every row sees.
+constexpr int kMinSplitBlocks = 4, kMinOlderBlocks = 8;
+
+__host__ __device__ inline int effective_splits(int S, int nbt, int nb0, int waves) {
+  if (waves == 4 && (nb0 == 0 || nb0 >= kMinOlderBlocks)) {
+    const int most = nbt / kMinSplitBlocks;
+    return most < 1 ? 1 : (S < most ? S : most);
+  }
+  int se = S < nb0 ? S : nb0;
+  while (se > 1 && (se - 1) * ((nbt + se - 1) / se) > nb0 - 1) --se;
+  return se < 1 ? 1 : se;
+}
+
 // Workgroup = NW waves x 16 * CG query rows (CG 16-column groups per wave).  K (bf16, from the caches)
 // and V (fp16, from the pre-pass) blocks go through a ring of kRing LDS buffers; two register
 // stage sets keep the global loads two steps ahead of their LDS store.  Step i (block i in
@@ -441,10 +458,8 @@ constexpr int kTileBuf = 1024;     // uint4 per block buffer (16 KiB)
 // The 2-wave instance (calls of at most 64 query rows per kv head, bound by HBM, not by the matrix
 // pipe) splits P into fp16 hi + lo and runs P V twice, so its probabilities carry ~22 bits
 // instead of 11.  prefill_tile runs query tile `tile` of (sequence b, kv head kvh), over key split
-// `split` of p.tile_splits: split s of S' covers blocks [s q, (s + 1) q), q = ceil(nbt / S'), the
-// last one to nbt, with S' <= S the most splits that all start in the older segment ((S' - 1) q <
-// nb0), so every split begins with an older block that every row sees (the exact maximum of its
-// first block is then finite for every row); splits from S' on are empty (their states say so).
+// `split` of p.tile_splits: split s of S' = effective_splits covers blocks [s q, (s + 1) q), q =
+// ceil(nbt / S'), the last one to nbt; splits from S' on are empty (their states say so).
 // kWide: the instance for tiles whose V does not fit fp16 (the pre-pass flagged one of their blocks):
 // V staged as bf16 from the caches (older blocks as bf16(V * s)), P split into bf16 hi + lo, P V and
 // the row sums on bf16 MFMAs; the fp16 instance skips those tiles and this one runs only them.
@@ -454,6 +469,7 @@ template <int NW, int CG, bool kPaged, bool kWide = false, int KS = 1>
 __device__ __attribute__((always_inline)) inline void prefill_tile(const PrefillParams& p, const int b, const int kvh,
                                                                    const int tile, const int split, uint4* lds) {
   constexpr bool kSplitP = NW == 2 || kWide;
+  constexpr bool kAnyStart = NW == 4 && !kWide;  // key splits may start where some rows see no key
   constexpr int kStages = 2;  // register stage sets (global loads run kStages steps ahead of their LDS store)
   constexpr int kDist = 2;    // step i stores block i + kDist into the LDS ring
   constexpr int kRing = kTileRing;
@@ -501,18 +517,15 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
   int kb0 = 0, kb1 = nbt;
   int steps = 0;  // the blocks of the longer half (both halves pass as many barriers)
   if (S > 1) {
-    // as many equal splits as start inside the older segment (a short older segment would leave
-    // the last split most of the keys: slower than no split)
-    int se = min(S, sv.nb0);
-    while (se > 1 && (se - 1) * ((nbt + se - 1) / se) > sv.nb0 - 1) --se;
-    const int q = (nbt + max(se, 1) - 1) / max(se, 1);
+    const int se = effective_splits(S, nbt, sv.nb0, NW);
+    const int q = (nbt + se - 1) / se;
     auto range = [&](int s) {
       int2 r = make_int2(0, nbt);
-      if (s >= max(se, 1)) {
+      if (s >= se) {
         r.y = 0;
       } else if (se > 1) {
-        r.x = s * q;
-        if (s + 1 < se) r.y = (s + 1) * q;
+        r.x = min(s * q, nbt);
+        if (s + 1 < se) r.y = min((s + 1) * q, nbt);  // (the last splits of q-block runs may come out empty)
       }
       return r;
     };
@@ -552,7 +565,8 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
 
   RowState rs[CG];
 #pragma unroll
-  for (int cg = 0; cg < CG; ++cg) rs[cg] = RowState{kNegInf, 0.f};
+  for (int cg = 0; cg < CG; ++cg)  // (rows past the end never wait for a key: see `unset`)
+    rs[cg] = RowState{kAnyStart && row0 + 16 * cg + n16 >= rows_total ? 0.f : kNegInf, 0.f};
   // O^T tiles (lane (n16, g4): dims 16 nb + 4 g4 + i of row n16) and the row sums of the fp16 P,
   // accumulated on the matrix pipe as P times a tile of ones (each lane holds its row's sum).
   f32x4 o[CG][8], ol[CG];
@@ -613,7 +627,9 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
       }
     }
     // Block 0 sets every row's reference to its exact maximum (a row that sees any key sees one
-    // in block 0: visible keys are a prefix of [older | local]).  Inside the loop the only rescale
+    // in block 0: visible keys are a prefix of [older | local]; a key split may start past a row's last
+    // key of its first block, and `unset` then sends the wave through the rescale branch until every
+    // row has a reference: the few blocks at the causal edge).  Inside the loop the only rescale
     // test is then the packed-probability overflow check, so the compiler keeps the QK^T MFMAs of
     // block i + 1 and the probabilities of block i in one scheduling region and interleaves them.
     {
@@ -633,6 +649,13 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
 #pragma unroll
       for (int cg = 0; cg < CG; ++cg) raise_rows(rs[cg], max8(s0[cg]), c, o[cg], ol[cg]);
     }
+    auto rows_unset = [&]() __attribute__((always_inline)) {
+      bool any = false;
+#pragma unroll
+      for (int cg = 0; cg < CG; ++cg) any |= rs[cg].m == kNegInf;
+      return __builtin_amdgcn_ballot_w64(any) != 0;
+    };
+    bool unset = kAnyStart && rows_unset();  // (wave-uniform)
 
     // Step i: the 16 LDS reads (K of block i + 1, V of block i) are issued first so their latency
     // passes under the mask work; then the QK^T MFMAs of block i + 1 are interleaved with the
@@ -712,7 +735,7 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
         __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);  // exp
       }
       // a new row maximum: exact maxima, rescale, recompute this block's P
-      if (__builtin_amdgcn_ballot_w64(kWide ? !(pmf < 512.f) : probs_overflow(pmax))) {
+      if (__builtin_amdgcn_ballot_w64(kWide ? !(pmf < 512.f) : probs_overflow(pmax)) != 0 || (kAnyStart && unset)) {
 #pragma unroll
         for (int cg = 0; cg < CG; ++cg) {
           raise_rows(rs[cg], max8(s[cg]), c, o[cg], ol[cg]);
@@ -725,6 +748,7 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
             if (kSplitP) probs_lo(pr, pw[cg], pl[cg]);
           }
         }
+        if (kAnyStart) unset = rows_unset();
       }
 #pragma unroll
       for (int nb = 0; nb < 8; ++nb)
@@ -1094,10 +1118,10 @@ namespace {
 // know how many of its sequences are long, and a step of decode rows and one or two prefill pieces
 // would leave half the CUs idle with 8-wave tiles) over a grid of at most ceil(T * G / rows_per_wg)
 // + B tiles per kv head.  A grid of fewer 4-wave workgroups than two per CU, or of 8-wave ones for
-// at most half the CUs, splits each tile's keys over up to 4 workgroups when the call has an older
-// segment and leaves the split counts to the library (num_splits 0): a 1024-token piece of one
-// sequence over 8K keys runs 256 4-wave workgroups, one wave per SIMD, and its key splits let a
-// second workgroup share each CU.
+// at most half the CUs, splits each tile's keys over up to 4 workgroups (8-wave tiles: when the call
+// has an older segment) when it leaves the split counts to the library (num_splits 0): a 1024-token
+// piece of one sequence over 8K keys has 256 4-wave tiles, one wave per SIMD, and its key splits put a
+// second wave on each.  lkv_prefill_attn then decides whether splits share workgroups.
 struct TilePlan {
   bool runs;          // the tile kernel runs (some sequence has > 64 rows per kv head, or tile_waves)
   int waves;
@@ -1134,7 +1158,7 @@ TilePlan tile_plan(const lkv_prefill_args* a) {
   const int64_t est = ragged ? ragged_tiles * a->num_kv_heads : t.wgs;  // the tiles that work
   // 4-wave tiles: below two workgroups per CU; 8-wave tiles (one per CU): at most half the CUs busy
   const bool idle = t.waves == 4 ? est < 2 * cus : (t.waves == 8 && est * 2 <= cus);
-  if (t.runs && idle && a->num_splits == 0 && a->older_k != nullptr && est > 0) {
+  if (t.runs && idle && a->num_splits == 0 && (a->older_k != nullptr || t.waves == 4) && est > 0) {
     // enough splits to fill the CUs' workgroup slots, rounded up to a power of two (a 768-token call
     // of one sequence, 32 query and 8 kv heads, over 8K keys: 192 4-wave tiles; 3 splits 156 us,
     // 4 splits 134 us, 2 splits 147 us)
@@ -1144,15 +1168,15 @@ TilePlan tile_plan(const lkv_prefill_args* a) {
     t.splits = static_cast<int>(std::min<int64_t>(kMaxTileSplits, pow2));
   }
   if (t.splits > 1 && a->older_len == nullptr && (a->local_k == nullptr || a->local_len == nullptr)) {
-    // host-constant lengths: as many equal splits as start inside the older segment for the last
-    // tile (the kernel applies the same rule per tile; a grid of splits that would all be empty
-    // would only cost their launch and the merge)
-    const int64_t nb0 = (std::min<int64_t>(std::max(a->older_len_const, 0), a->older_capacity_tokens) + kBlockTokens - 1) /
-                        kBlockTokens;
-    const int64_t lead = a->local_start ? kBlockTokens - 1 : (a->local_start_const & (kBlockTokens - 1));
-    const int64_t n1 = a->local_k == nullptr ? 0 : std::max(a->local_len_const, 0);
-    const int64_t nbt = nb0 + (n1 > 0 ? (lead + n1 + kBlockTokens - 1) / kBlockTokens : 0);
-    while (t.splits > 1 && (t.splits - 1) * ((nbt + t.splits - 1) / t.splits) > nb0 - 1) --t.splits;
+    // host-constant lengths: the splits the last tile takes (the kernel applies the same rule per tile; a
+    // grid of splits that would all be empty would only cost their launch and the merge)
+    const int nb0 = a->older_k == nullptr
+                        ? 0
+                        : (std::min<int>(std::max(a->older_len_const, 0), a->older_capacity_tokens) + kBlockTokens - 1) / kBlockTokens;
+    const int lead = a->local_start ? kBlockTokens - 1 : (a->local_start_const & (kBlockTokens - 1));
+    const int n1 = a->local_k == nullptr ? 0 : std::max(a->local_len_const, 0);
+    const int nbt = nb0 + (n1 > 0 ? (lead + n1 + kBlockTokens - 1) / kBlockTokens : 0);
+    t.splits = effective_splits(t.splits, nbt, nb0, t.waves);
   }
   return t;
 }
@@ -1421,18 +1445,32 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
   const int waves = plan.waves;
   const int64_t tiles = plan.tiles, wgs = plan.wgs;
   LKV_REQUIRE((mixed ? mixed_grid(rows16.items, wgs * splits) : wgs * splits) < (1LL << 31), "too many query rows");
-  // Pairs of 4-wave key splits share a workgroup of 8 waves and merge in LDS, when half as many workgroups
-  // still fill the CUs (at least 3/4 of the rounds they take): the states' round trip through memory and,
-  // for 2 splits, the merge launch go.  One sequence's 1024 tokens at 7K (256 tiles, 2 splits) 152.4 ->
-  // 140.3 us, 1000 at 3K 127.5 -> 116.0, 512 at 8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line 200
-  // tokens at 5K (56 tiles, 4 splits) would take 59.5 instead of 51.3 and two sequences' 300 at 3K (160
-  // tiles, 4 splits: 320 workgroups, a second round of 64) 81.6 instead of 78.0.  Uniform calls only: a
-  // ragged call's tiles keep one arithmetic whether or not they share a launch with decode rows.
+  // Workgroups of 8 waves whose two halves take a key half each and merge in LDS, in place of 4-wave tiles
+  // with key splits:
+  // - a grid of at most half the CUs takes as many splits as leave one such workgroup per CU, each in two
+  //   halves (two waves per SIMD where 4-wave tiles leave one): one sequence's 20 tokens at 2K 56.8 -> 30.8
+  //   us, 200 at 5K 51.4 -> 44.4, 40 at 5K (paged) 84.4 -> 43.5, 150 tokens of 8 heads without groups at 16K
+  //   102 -> 84 (with splits that may start in the local segment, effective_splits);
+  // - else an even number of splits runs as pairs, when half as many workgroups still fill the CUs (at least
+  //   3/4 of the rounds they take): the states' round trip through memory and, for 2 splits, the merge
+  //   launch go.  1024 tokens at 7K (256 tiles, 2 splits) 152.4 -> 139 us, 1000 at 3K 127.5 -> 116.0, 512 at
+  //   8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line two sequences' 300 at 3K (160 tiles, 4 splits: 320
+  //   workgroups, a second round of 64) would take 81.6 instead of 78.0.
+  // Uniform calls only: a ragged call's tiles keep one arithmetic whether or not they share a launch with
+  // decode rows.
   const int64_t cu_count = device_cu_count() > 0 ? device_cu_count() : 256;
-  const int64_t half_wgs = wgs * splits / 2;
-  const bool halves = waves == 4 && splits % 2 == 0 && !ragged && half_wgs >= cu_count &&
-                      half_wgs * 4 >= (half_wgs + cu_count - 1) / cu_count * cu_count * 3;
-  if (halves) splits /= 2;
+  bool halves = false;
+  if (waves == 4 && splits > 1 && !ragged) {
+    const int64_t half_wgs = wgs * splits / 2;
+    if (2 * wgs <= cu_count && vblocks >= 2 * splits * kMinSplitBlocks) {
+      splits = static_cast<int>(std::min<int64_t>(splits, cu_count / wgs));
+      halves = true;
+    } else if (splits % 2 == 0 && half_wgs >= cu_count &&
+               half_wgs * 4 >= (half_wgs + cu_count - 1) / cu_count * cu_count * 3) {
+      splits /= 2;
+      halves = true;
+    }
+  }
   p.tile_splits = splits;
   p.ws_o = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(a->workspace) + v16_bytes) : nullptr;
   p.ws_lse = splits > 1 ? p.ws_o + plan.rows_all * a->num_q_heads * splits * kHeadDim : nullptr;

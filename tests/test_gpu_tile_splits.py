@@ -145,3 +145,57 @@ def test_key_halves_of_one_workgroup_match_oracle(T0, L, causal, wide, paged):
         torch.testing.assert_close(lse[0, :, h].double(), torch.logsumexp(s, -1), rtol=1e-4, atol=1e-4)
         want = want.bfloat16().double()
         assert float((got[0, :, h].double() - want).norm() / want.norm()) <= REL_L2
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("T0,n1,L,Hkv,G,shift", [(0, 1200, 100, 2, 4, 0.0), (0, 1201, 130, 3, 1, 8.0), (256, 900, 70, 1, 7, 8.0),
+                                                 (640, 1500, 257, 2, 2, 8.0), (1024, 33, 33, 2, 4, 8.0), (0, 129, 129, 2, 1, 8.0)])
+def test_key_splits_that_start_in_the_local_segment(T0, n1, L, Hkv, G, shift, paged):
+    """Few tiles over a short (or no) older segment: key splits start in the causal local segment, so rows see
+    no key in their split's first block (or in any of its blocks), row tiles end in padding, and halves get
+    unequal blocks.  With ``shift`` every score sits near -90 (2^-130 against a zero reference: a row whose
+    reference were not taken from the first block it sees would lose all of its probabilities)."""
+
+    g = torch.Generator(device=DEV).manual_seed(T0 + n1 + L)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device=DEV)  # noqa: E731
+    u = rnd(128)
+    u = u / u.norm() * 128 ** 0.5
+    q = (rnd(1, L, Hkv * G, 128) - shift * u).bfloat16()
+    k = ((0.2 if shift else 1.0) * rnd(1, Hkv, T0 + n1, 128) + (u if shift else 0.0)).bfloat16()
+    v = rnd(1, Hkv, T0 + n1, 128).bfloat16()
+    R = -(-n1 // 32) * 32 + 64
+    start = 45
+    if paged:
+        blocks = max(1, T0 // 32) + R // 32
+        pool = ops.PagedKV.zeros(blocks, Hkv, DEV)
+        table = torch.randperm(blocks, generator=torch.Generator().manual_seed(1)).to(DEV, torch.int32)[None]
+        ot, rt = table[:, :max(1, T0 // 32)], table[:, max(1, T0 // 32):]
+        if T0:
+            ops.append_paged(k[:, :, :T0].transpose(1, 2), v[:, :, :T0].transpose(1, 2), pool, ot, token0=0)
+        ops.append_paged(k[:, :, T0:].transpose(1, 2), v[:, :, T0:].transpose(1, 2), pool, rt, token0=start, wrap_tokens=R)
+        i32 = lambda x: torch.tensor([x], dtype=torch.int32, device=DEV)  # noqa: E731
+        seg = dict(older=pool, older_table=ot, older_len=i32(T0), local=pool, local_table=rt, local_len=i32(n1),
+                   local_start=i32(start))
+    else:
+        ring = ops.TiledKV.zeros(1, Hkv, R, DEV)
+        first = min(n1, R - start)
+        ops.pack_kv(k[:, :, T0:T0 + first], v[:, :, T0:T0 + first], ring, token0=start)
+        if first < n1:
+            ops.pack_kv(k[:, :, T0 + first:], v[:, :, T0 + first:], ring, token0=0)
+        seg = dict(local=ring, local_len=n1, local_start=start)
+        if T0:
+            older = ops.TiledKV.zeros(1, Hkv, T0, DEV)
+            ops.pack_kv(k[:, :, :T0], v[:, :, :T0], older)
+            seg.update(older=older, older_len=T0)
+    lse = torch.empty((1, L, Hkv * G), dtype=torch.float32, device=DEV)
+    got = ops.prefill_attention(q, causal=True, lse=lse, tile_waves=4, **seg)[0].float()
+    n = T0 + n1
+    hide = torch.arange(n, device=DEV)[None, :] > (n - L + torch.arange(L, device=DEV))[:, None]
+    want = torch.empty(L, Hkv * G, 128, dtype=torch.float64, device=DEV)
+    for h in range(Hkv * G):
+        s = (q[0, :, h].double() @ k[0, h // G].double().t().contiguous() / 128 ** 0.5).masked_fill(hide, float("-inf"))
+        torch.testing.assert_close(lse[0, :, h].double(), torch.logsumexp(s, -1), rtol=1e-4, atol=1e-4)
+        want[:, h] = torch.softmax(s, -1) @ v[0, h // G].double()
+    want = want.bfloat16().double()
+    assert float((got.double() - want).norm() / want.norm()) <= REL_L2
+    assert float((got.double() - want).abs().max()) <= MAX_ABS
