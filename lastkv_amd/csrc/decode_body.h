@@ -34,6 +34,7 @@ struct DecodeParams {
   const int32_t* cu;
   int32_t rows, col_lo, col_hi;
   int32_t dyn_splits, cus, lmax;
+  int32_t interleave;  // key splits take interleaved blocks (large tiled calls) instead of contiguous ranges
 };
 
 // Query tokens of sequence b (kMulti calls) and the flattened row of its token 0 (the q / out / lse
@@ -301,12 +302,17 @@ __device__ __attribute__((always_inline)) inline void decode_split_body(const De
 
   const SeqView sv = make_seq_view(p.seg, b, kvh);
   const int nbt = sv.nb0 + (sv.n1 > 0 ? (sv.lead + sv.n1 + kBlockTokens - 1) / kBlockTokens : 0);
-  // Splits interleave: wave w of split s takes blocks s * kStride + w, + S * kStride, ..., so that the
-  // workgroups of one (sequence, kv head) walk one window of its K and V together: fewer DRAM pages are
-  // open at once than with a contiguous range per split (the same box, 128K keys: 4 sequences 330 -> 318
-  // us, 2 sequences 190 -> 168, one 100 -> 87; 8 sequences at 8.3K 46.6 -> 45.3), and the ring's ragged
-  // blocks spread over all splits.
-  const int step = S * kStride;
+  // Large calls over tiled caches interleave their splits: wave w of split s takes blocks s * kStride + w, + S * kStride, ...,
+  // so that the workgroups of one (sequence, kv head) walk one window of its K and V together: fewer DRAM
+  // pages are open at once than with a contiguous range per split (128K keys: 4 sequences 330 -> 318 us, 2
+  // sequences 190 -> 168, one 100 -> 87).  Below 384 MiB of K/V, which the last-level cache partly holds,
+  // ranges were up to 4 % faster (7 sequences at 16K, 4 kv heads: 47.4 against 49.2 us), as they were for
+  // paged segments (9 sequences at 16K: 104.6 against 107.3), whose page ids would then come from another
+  // cache line of the table for every block.
+  const int bps = (nbt + S - 1) / S;
+  const int step = p.interleave ? S * kStride : kStride;
+  const int blk_begin = p.interleave ? split * kStride : split * bps;
+  const int blk_end = p.interleave ? nbt : min(blk_begin + bps, nbt);
 
   const int cols = kMulti ? G * Lq : G;
   uint4 qf[CG][4];
@@ -343,15 +349,15 @@ __device__ __attribute__((always_inline)) inline void decode_split_body(const De
   // this wave's blocks: first + step * t, t < nw; block t + 1 is loaded while block t is computed.  The
   // loop runs while two or more blocks remain, so its loads are unconditional (the compiler then counts
   // them exactly for s_waitcnt); the last one or two blocks follow it.
-  const int first = split * kStride + (kPairs ? (wave & 1) : wave);
-  if (first < nbt) {
-    int nw = (nbt - 1 - first) / step + 1;
+  const int first = blk_begin + (kPairs ? (wave & 1) : wave);
+  if (first < blk_end) {
+    int nw = (blk_end - 1 - first) / step + 1;
     // A wave with one block more than the workgroup's last wave (the split's block count is not a
     // multiple of the waves) fetches that last block together with its first one and computes it
     // after the loop, so its extra block adds compute but no round trip to memory: the loop, whose
     // iterations are bound by load latency, then runs as many iterations in every wave.
-    const int last_first = split * kStride + kStride - 1;
-    const int nw_last = last_first < nbt ? (nbt - 1 - last_first) / step + 1 : 0;
+    const int last_first = blk_begin + kStride - 1;
+    const int nw_last = last_first < blk_end ? (blk_end - 1 - last_first) / step + 1 : 0;
     const bool fold = kFold && nw > nw_last && nw >= 2;
     BlockFrags fa, fb, fc;
     BlockRef ra = block_ref(sv, first), rc{};

@@ -1159,13 +1159,16 @@ TilePlan tile_plan(const lkv_prefill_args* a) {
   // 4-wave tiles: below two workgroups per CU; 8-wave tiles (one per CU): at most half the CUs busy
   const bool idle = t.waves == 4 ? est < 2 * cus : (t.waves == 8 && est * 2 <= cus);
   if (t.runs && idle && a->num_splits == 0 && (a->older_k != nullptr || t.waves == 4) && est > 0) {
-    // enough splits to fill the CUs' workgroup slots, rounded up to a power of two (a 768-token call
-    // of one sequence, 32 query and 8 kv heads, over 8K keys: 192 4-wave tiles; 3 splits 156 us,
-    // 4 splits 134 us, 2 splits 147 us)
-    int64_t want = (cus * (t.waves == 4 ? 2 : 1) + est - 1) / est;
-    int64_t pow2 = 1;
-    while (pow2 < want) pow2 *= 2;
-    t.splits = static_cast<int>(std::min<int64_t>(kMaxTileSplits, pow2));
+    // as many splits as run in one round of the CUs' workgroup slots; where that is 2 and leaves an eighth of
+    // them empty, 4 in two rounds (768 tokens of one sequence at 8K, 192 4-wave tiles: 4 splits 134 us, 3
+    // splits 156, 2 splits 147; four sequences' 200 tokens at 3K, 224 tiles: 2 splits 84.6, 4 splits 90.4;
+    // nine of 55 tokens at 4K, 144 tiles: 3 splits 88.4, 4 splits 100.6); a grid of more than half the
+    // slots takes 2 while an eighth of them would stay empty
+    const int64_t slots = cus * (t.waves == 4 ? 2 : 1);
+    const int64_t one = slots / est;
+    int64_t n = one;
+    if (one <= 2) n = one * est * 8 >= slots * 7 ? one : 2 * one;
+    t.splits = static_cast<int>(std::min<int64_t>(kMaxTileSplits, n));
   }
   if (t.splits > 1 && a->older_len == nullptr && (a->local_k == nullptr || a->local_len == nullptr)) {
     // host-constant lengths: the splits the last tile takes (the kernel applies the same rule per tile; a
@@ -1451,11 +1454,11 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
   //   halves (two waves per SIMD where 4-wave tiles leave one): one sequence's 20 tokens at 2K 56.8 -> 30.8
   //   us, 200 at 5K 51.4 -> 44.4, 40 at 5K (paged) 84.4 -> 43.5, 150 tokens of 8 heads without groups at 16K
   //   102 -> 84 (with splits that may start in the local segment, effective_splits);
-  // - else an even number of splits runs as pairs, when half as many workgroups still fill the CUs (at least
-  //   3/4 of the rounds they take): the states' round trip through memory and, for 2 splits, the merge
+  // - else an even number of splits runs as pairs, when half as many workgroups still fill the CUs (more than
+  //   7/8 of the rounds they take): the states' round trip through memory and, for 2 splits, the merge
   //   launch go.  1024 tokens at 7K (256 tiles, 2 splits) 152.4 -> 139 us, 1000 at 3K 127.5 -> 116.0, 512 at
   //   8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line two sequences' 300 at 3K (160 tiles, 4 splits: 320
-  //   workgroups, a second round of 64) would take 81.6 instead of 78.0.
+  //   workgroups, a second round of 64) would take 81.6 instead of 78.0, six of 100 at 5K (384) 128.9 of 116.
   // Uniform calls only: a ragged call's tiles keep one arithmetic whether or not they share a launch with
   // decode rows.
   const int64_t cu_count = device_cu_count() > 0 ? device_cu_count() : 256;
@@ -1466,7 +1469,7 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
       splits = static_cast<int>(std::min<int64_t>(splits, cu_count / wgs));
       halves = true;
     } else if (splits % 2 == 0 && half_wgs >= cu_count &&
-               half_wgs * 4 >= (half_wgs + cu_count - 1) / cu_count * cu_count * 3) {
+               half_wgs * 8 > (half_wgs + cu_count - 1) / cu_count * cu_count * 7) {
       splits /= 2;
       halves = true;
     }
