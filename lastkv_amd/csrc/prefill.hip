@@ -844,12 +844,13 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
       const int tok = row / G, h = row - tok * G;
       const int64_t srow = ((sr.lse0 + tok) * p.hq + kvh * G + h) * p.tile_splits + (kWide ? 0 : split);
       float* orow = p.ws_o + srow * kHeadDim;
-      if (lt > 0.f) {  // (an empty split's O is never read: its LSE says so)
+      const bool some = !(lt <= 0.f);  // (a NaN sum is a state too: the row's result is NaN)
+      if (some) {  // (an empty split's O has no weight: its LSE says so)
 #pragma unroll
         for (int nb = 0; nb < 8; ++nb)
           *reinterpret_cast<f32x4*>(orow + 16 * nb + 4 * g4) = o[cg][nb] * linv;
       }
-      if (g4 == 0) p.ws_lse[srow] = lt > 0.f ? rs[cg].mc + __log2f(lt) : kNegInf;
+      if (g4 == 0) p.ws_lse[srow] = some ? rs[cg].mc + __log2f(lt) : kNegInf;
       if (kWide && g4 < p.tile_splits - 1) p.ws_lse[srow + 1 + g4] = kNegInf;  // (the other splits, <= 3: empty)
     } else if (row < rows_total) {
       const int tok = row / G, h = row - tok * G;
@@ -1034,15 +1035,13 @@ __global__ __launch_bounds__(256) void prefill_split_combine_kernel(const Prefil
 #pragma unroll
   for (int s = 0; s < kMaxTileSplits; ++s) m = fmaxf(m, ls[s]);
   float l = 0.f, o0 = 0.f, o1 = 0.f;
-  if (m != kNegInf) {
 #pragma unroll
-    for (int s = 0; s < kMaxTileSplits; ++s) {
-      if (ls[s] == kNegInf) continue;  // (no visible key, or no such split: weight 0)
-      const float w = fast_exp2(ls[s] - m);
-      l += w;
-      o0 += w * x[s].x;
-      o1 += w * x[s].y;
-    }
+  for (int s = 0; s < kMaxTileSplits; ++s) {
+    if (ls[s] == kNegInf) continue;  // (no visible key, or no such split: weight 0)
+    const float w = fast_exp2(ls[s] - m);  // (NaN for a NaN state, also where no split has a finite one)
+    l += w;
+    o0 += w * x[s].x;
+    o1 += w * x[s].y;
   }
   const float linv = l > 0.f ? 1.f / l : 0.f;
   uint32_t w01 = pack_bf16x2(o0 * linv, o1 * linv);

@@ -199,3 +199,29 @@ def test_key_splits_that_start_in_the_local_segment(T0, n1, L, Hkv, G, shift, pa
     want = want.bfloat16().double()
     assert float((got.double() - want).norm() / want.norm()) <= REL_L2
     assert float((got.double() - want).abs().max()) <= MAX_ABS
+
+
+@pytest.mark.parametrize("B,L,T0,tile_waves", [(1, 40, 1500, 4), (1, 512, 1500, 0), (2, 300, 1500, 0), (1, 130, 0, 4)])
+def test_a_nan_key_reaches_every_row_that_sees_it(B, L, T0, tile_waves):
+    """One NaN key in the local segment: exactly the rows that see it are NaN, with key splits (as halves of a
+    workgroup, as states in memory, or both) as without, whichever split holds the key."""
+
+    g = torch.Generator(device=DEV).manual_seed(B + L + T0)
+    Hkv, G, n1 = 8, 4, L + 300
+    rnd = lambda *shape: torch.randn(shape, generator=g, device=DEV).bfloat16()  # noqa: E731
+    q, lk, lv = rnd(B, L, Hkv * G, 128), rnd(B, Hkv, n1, 128), rnd(B, Hkv, n1, 128)
+    ring = ops.TiledKV.zeros(B, Hkv, -(-n1 // 32) * 32, DEV)
+    seg = dict(local=ring, local_len=n1)
+    if T0:
+        older = ops.TiledKV.zeros(B, Hkv, -(-T0 // 32) * 32, DEV)
+        ops.pack_kv(rnd(B, Hkv, T0, 128), rnd(B, Hkv, T0, 128), older)
+        seg.update(older=older, older_len=T0)
+    for at in (0, 299, n1 - 5, n1 - 1):  # (query row r sees keys up to r + 300)
+        bad = lk.clone()
+        bad[0, 1, at] = float("nan")
+        ops.pack_kv(bad, lv, ring)
+        want = torch.zeros(B, L, Hkv * G, 128, dtype=torch.bool, device=DEV)
+        want[0, max(0, at - 300):, G:2 * G] = True
+        for splits in (0, 1):
+            got = ops.prefill_attention(q, causal=True, tile_waves=tile_waves, num_splits=splits, **seg)
+            assert torch.equal(torch.isnan(got), want), f"key {at}, num_splits {splits}"
