@@ -220,8 +220,10 @@ struct RowState {
 
 // Raises each row's reference to its maximum over this block (lm = lane maxima) and rescales O
 // and the row sums by 2^(mc_old - mc_new).  Runs for the first block and in a wave-uniform branch
-// taken whenever some P reached 2^9.
-__device__ inline void raise_rows(RowState& rs, float lm, float c, f32x4 (&o)[8], f32x4& ol) {
+// taken whenever some P reached 2^9.  unset: mc of a row that has seen no key (with kUnset its first
+// key's P overflows, so that the branch gives the row its reference).
+constexpr float kUnset = -1e30f;
+__device__ inline void raise_rows(RowState& rs, float lm, float c, f32x4 (&o)[8], f32x4& ol, float unset = 0.f) {
   const float bm = wave_max_across_rows(lm);
   const bool up = bm > rs.m;  // m = -inf: true for the first finite maximum
   const float mc_new = up ? bm * c : rs.mc;
@@ -229,7 +231,7 @@ __device__ inline void raise_rows(RowState& rs, float lm, float c, f32x4 (&o)[8]
   // (and 0 * inf = NaN) when the first maximum is below -128 / c
   const float alpha = up ? (rs.m == kNegInf ? 0.f : fast_exp2(rs.mc - mc_new)) : 1.f;
   rs.m = up ? bm : rs.m;
-  rs.mc = rs.m == kNegInf ? 0.f : mc_new;
+  rs.mc = rs.m == kNegInf ? unset : mc_new;
   if (__builtin_amdgcn_ballot_w64(alpha != 1.f)) {
 #pragma unroll
     for (int nb = 0; nb < 8; ++nb) o[nb] *= alpha;
@@ -470,6 +472,7 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
                                                                    const int tile, const int split, uint4* lds) {
   constexpr bool kSplitP = NW == 2 || kWide;
   constexpr bool kAnyStart = NW == 4 && !kWide;  // key splits may start where some rows see no key
+  constexpr float kUnsetMc = kAnyStart ? kUnset : 0.f;
   constexpr int kStages = 2;  // register stage sets (global loads run kStages steps ahead of their LDS store)
   constexpr int kDist = 2;    // step i stores block i + kDist into the LDS ring
   constexpr int kRing = kTileRing;
@@ -565,7 +568,7 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
 
   RowState rs[CG];
 #pragma unroll
-  for (int cg = 0; cg < CG; ++cg)  // (rows past the end never wait for a key: see `unset`)
+  for (int cg = 0; cg < CG; ++cg)  // (rows past the end never take a first key's branch)
     rs[cg] = RowState{kAnyStart && row0 + 16 * cg + n16 >= rows_total ? 0.f : kNegInf, 0.f};
   // O^T tiles (lane (n16, g4): dims 16 nb + 4 g4 + i of row n16) and the row sums of the fp16 P,
   // accumulated on the matrix pipe as P times a tile of ones (each lane holds its row's sum).
@@ -628,8 +631,8 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
     }
     // Block 0 sets every row's reference to its exact maximum (a row that sees any key sees one
     // in block 0: visible keys are a prefix of [older | local]; a key split may start past a row's last
-    // key of its first block, and `unset` then sends the wave through the rescale branch until every
-    // row has a reference: the few blocks at the causal edge).  Inside the loop the only rescale
+    // key of its first block, and the row's reference kUnset then sends the wave through the rescale
+    // branch at the row's first key: the few blocks at the causal edge).  Inside the loop the only rescale
     // test is then the packed-probability overflow check, so the compiler keeps the QK^T MFMAs of
     // block i + 1 and the probabilities of block i in one scheduling region and interleaves them.
     {
@@ -647,15 +650,8 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
         for (int cg = 0; cg < CG; ++cg) mask_scores(s0[cg], r0, lim[cg], g4);
       }
 #pragma unroll
-      for (int cg = 0; cg < CG; ++cg) raise_rows(rs[cg], max8(s0[cg]), c, o[cg], ol[cg]);
+      for (int cg = 0; cg < CG; ++cg) raise_rows(rs[cg], max8(s0[cg]), c, o[cg], ol[cg], kUnsetMc);
     }
-    auto rows_unset = [&]() __attribute__((always_inline)) {
-      bool any = false;
-#pragma unroll
-      for (int cg = 0; cg < CG; ++cg) any |= rs[cg].m == kNegInf;
-      return __builtin_amdgcn_ballot_w64(any) != 0;
-    };
-    bool unset = kAnyStart && rows_unset();  // (wave-uniform)
 
     // Step i: the 16 LDS reads (K of block i + 1, V of block i) are issued first so their latency
     // passes under the mask work; then the QK^T MFMAs of block i + 1 are interleaved with the
@@ -735,10 +731,10 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
         __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);  // exp
       }
       // a new row maximum: exact maxima, rescale, recompute this block's P
-      if (__builtin_amdgcn_ballot_w64(kWide ? !(pmf < 512.f) : probs_overflow(pmax)) != 0 || (kAnyStart && unset)) {
+      if (__builtin_amdgcn_ballot_w64(kWide ? !(pmf < 512.f) : probs_overflow(pmax)) != 0) {
 #pragma unroll
         for (int cg = 0; cg < CG; ++cg) {
-          raise_rows(rs[cg], max8(s[cg]), c, o[cg], ol[cg]);
+          raise_rows(rs[cg], max8(s[cg]), c, o[cg], ol[cg], kUnsetMc);
           if constexpr (kWide) {
             float pm;
             probs_bf16(s[cg], c, rs[cg].mc, pw[cg], pl[cg], pm);
@@ -748,7 +744,6 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
             if (kSplitP) probs_lo(pr, pw[cg], pl[cg]);
           }
         }
-        if (kAnyStart) unset = rows_unset();
       }
 #pragma unroll
       for (int nb = 0; nb < 8; ++nb)
