@@ -568,8 +568,7 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
 
   RowState rs[CG];
 #pragma unroll
-  for (int cg = 0; cg < CG; ++cg)  // (rows past the end never take a first key's branch)
-    rs[cg] = RowState{kAnyStart && row0 + 16 * cg + n16 >= rows_total ? 0.f : kNegInf, 0.f};
+  for (int cg = 0; cg < CG; ++cg) rs[cg] = RowState{kNegInf, 0.f};
   // O^T tiles (lane (n16, g4): dims 16 nb + 4 g4 + i of row n16) and the row sums of the fp16 P,
   // accumulated on the matrix pipe as P times a tile of ones (each lane holds its row's sum).
   f32x4 o[CG][8], ol[CG];
@@ -946,7 +945,7 @@ __global__ __launch_bounds__(NW * KS * 64) __attribute__((amdgpu_waves_per_eu(WP
 // kMixRun workgroups (the dispatcher deals workgroups to the XCDs, their shader engines and CUs in turn, so
 // half of every engine's CUs take decode items, two each, and the other half tiles); the remaining tiles
 // follow and take the CUs of the decode items that end.  31 decode rows at 8K, a 1024-token row and a
-// 7-token row: the step 374 -> 325 us; runs of 32 to 128 alike, runs of 256 (a decode item beside a tile on
+// 7-token row: the step 374 -> 322 us; runs of 32 to 128 alike, runs of 256 (a decode item beside a tile on
 // every CU) 366, of 8 (whole shader engines of one kind) 395, decode items first 367.
 constexpr int kMixRun = 64;
 
@@ -1446,11 +1445,11 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
   // with key splits:
   // - a grid of at most half the CUs takes as many splits as leave one such workgroup per CU, each in two
   //   halves (two waves per SIMD where 4-wave tiles leave one): one sequence's 20 tokens at 2K 56.8 -> 30.8
-  //   us, 200 at 5K 51.4 -> 44.4, 40 at 5K (paged) 84.4 -> 43.5, 150 tokens of 8 heads without groups at 16K
+  //   us, 200 at 5K 51.4 -> 44.4, 40 at 5K (paged) 84.4 -> 41.3, 150 tokens of 8 heads without groups at 16K
   //   102 -> 84 (with splits that may start in the local segment, effective_splits);
   // - else an even number of splits runs as pairs, when half as many workgroups still fill the CUs (more than
   //   7/8 of the rounds they take): the states' round trip through memory and, for 2 splits, the merge
-  //   launch go.  1024 tokens at 7K (256 tiles, 2 splits) 152.4 -> 139 us, 1000 at 3K 127.5 -> 116.0, 512 at
+  //   launch go.  1024 tokens at 7K (256 tiles, 2 splits) 152.4 -> 136 us, 1000 at 3K 127.5 -> 116.0, 512 at
   //   8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line two sequences' 300 at 3K (160 tiles, 4 splits: 320
   //   workgroups, a second round of 64) would take 81.6 instead of 78.0, six of 100 at 5K (384) 128.9 of 116.
   // Uniform calls only: a ragged call's tiles keep one arithmetic whether or not they share a launch with
