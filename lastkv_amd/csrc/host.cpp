@@ -3,9 +3,11 @@
 // Each function takes the positional arguments of the ops function of the same name, applies that
 // function's checks to the common forms of the arguments (exact torch tensors with storage on a GPU,
 // Python ints, TiledKV / PagedKV segments), fills the C-ABI struct and calls the library.  It returns
-// the output tensor, or None when an argument has another form, a check fails or the library returns
-// an error: ops.py then runs its own path, which handles the rest and raises the errors.  Nothing is
-// kept between calls but the library's entry points and each device's CU count.
+// the output tensor, or None when an argument has another form, a check fails or the library refuses the
+// arguments: ops.py then runs its own path, which handles the rest and raises the errors.  An error of the
+// HIP runtime raises here: the library reports it after a launch (it may be an older one that the launch
+// only found), and the call's work must not be issued again.  Nothing is kept between calls but the
+// library's entry points and each device's CU count.
 //
 // What bounds it: a decode or epilogue call of a few sequences is 5-10 us of GPU time, and the Python
 // path took 20-35 us to issue it (attribute reads of ~20 tensors, ~45 ctypes field stores); here 5-9 us
@@ -34,11 +36,13 @@ struct Library {
   decltype(&lkv_qkv_epilogue) qkv_epilogue;
   decltype(&lkv_rmsnorm) rmsnorm;
   decltype(&lkv_silu_mul) silu_mul;
+  decltype(&lkv_last_error) last_error;
 };
 
 Library g_lib;
 PyTypeObject* g_tiled = nullptr;
 PyTypeObject* g_paged = nullptr;
+PyObject* g_error = nullptr;  // LastKVNativeError
 PyObject* g_str_k = nullptr;
 PyObject* g_str_v = nullptr;
 constexpr int kMaxDevices = 64;
@@ -247,7 +251,20 @@ int32_t without_gil(F&& f) {
   Py_END_ALLOW_THREADS return st;
 }
 
-// Runs f, which returns a new reference; a C++ exception (an allocation that fails, say) is left to the
+// Calls the library and returns the call's result (made first, so that nothing can fail after a launch): the
+// output, None for arguments it refuses, or null with the error set for one of the HIP runtime.
+template <class F>
+PyObject* issue(const char* what, PyObject* given, const at::Tensor& out, F&& call) {
+  PyObject* r = result(given, out);
+  if (r == nullptr) return nullptr;
+  const int32_t st = without_gil(call);
+  if (st == LKV_OK) return r;
+  Py_DECREF(r);
+  if (st != LKV_ERR_HIP) return not_handled();
+  return PyErr_Format(g_error, "%s failed (status %d): %s", what, static_cast<int>(st), g_lib.last_error());
+}
+
+// Runs f, which returns a new reference or null with an error set; a C++ exception (an allocation that fails, say) is left to the
 // Python path to meet again and report.
 template <class F>
 PyObject* guarded(F&& f) {
@@ -330,8 +347,7 @@ PyObject* decode_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
     a.workspace = ws.defined() ? ptr(ws) : nullptr;
     a.workspace_bytes = ws.defined() ? static_cast<int64_t>(ws.nbytes()) : 0;
     const lkv_stream_t s = stream_of(*q);
-    if (without_gil([&] { return g_lib.decode_attn(&a, s); }) != LKV_OK) return not_handled();
-    return result(v[14], out);
+    return issue("lkv_decode_attn", v[14], out, [&] { return g_lib.decode_attn(&a, s); });
   });
 }
 
@@ -421,14 +437,15 @@ PyObject* prefill_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
     } else {
       ws = new_bytes(std::max<int64_t>(16, g_lib.prefill_workspace_bytes(&a)), dev);
     }
+    PyObject* done = nullptr;
     if (ok) {
       a.workspace = ptr(ws);
       a.workspace_bytes = static_cast<int64_t>(ws.nbytes());
       const lkv_stream_t s = stream_of(*q);
-      ok = without_gil([&] { return g_lib.prefill_attn(&a, s); }) == LKV_OK;
+      done = issue("lkv_prefill_attn", v[14], out, [&] { return g_lib.prefill_attn(&a, s); });
     }
     if (host.obj != nullptr) PyBuffer_Release(&host);
-    return ok ? result(v[14], out) : not_handled();
+    return ok ? done : not_handled();
   });
 }
 
@@ -569,8 +586,7 @@ PyObject* qkv_epilogue(PyObject*, PyObject* const* v, Py_ssize_t n) {
         return not_handled();
     }
     const lkv_stream_t s = stream_of(*q);
-    if (without_gil([&] { return g_lib.qkv_epilogue(&a, s); }) != LKV_OK) return not_handled();
-    return result(v[15], out);
+    return issue("lkv_qkv_epilogue", v[15], out, [&] { return g_lib.qkv_epilogue(&a, s); });
   });
 }
 
@@ -625,8 +641,8 @@ PyObject* rmsnorm(PyObject*, PyObject* const* v, Py_ssize_t n) {
     a.weight = ptr(*w);
     a.out = ptr(out);
     const lkv_stream_t s = stream_of(*x);
-    if (nrows > INT32_MAX || without_gil([&] { return g_lib.rmsnorm(&a, s); }) != LKV_OK) return not_handled();
-    return result(v[4], out);
+    if (nrows > INT32_MAX) return not_handled();
+    return issue("lkv_rmsnorm", v[4], out, [&] { return g_lib.rmsnorm(&a, s); });
   });
 }
 
@@ -648,19 +664,19 @@ PyObject* silu_mul(PyObject*, PyObject* const* v, Py_ssize_t n) {
     }
     const lkv_stream_t s = stream_of(*g);
     if (nrows > INT32_MAX || width > INT32_MAX) return not_handled();
-    if (without_gil([&] {
-          return g_lib.silu_mul(ptr(*g), gs, ptr(*u), us, ptr(out), os, static_cast<int32_t>(nrows),
-                                static_cast<int32_t>(width), s);
-        }) != LKV_OK)
-      return not_handled();
-    return result(v[2], out);
+    return issue("lkv_silu_mul", v[2], out, [&] {
+      return g_lib.silu_mul(ptr(*g), gs, ptr(*u), us, ptr(out), os, static_cast<int32_t>(nrows), static_cast<int32_t>(width),
+                            s);
+    });
   });
 }
 
-// bind(addresses: the entry points in Library's order, TiledKV, PagedKV)
+// bind(addresses: the entry points in Library's order, TiledKV, PagedKV, LastKVNativeError)
 PyObject* bind(PyObject*, PyObject* args) {
-  PyObject *addresses, *tiled, *paged;
-  if (!PyArg_ParseTuple(args, "O!O!O!", &PyTuple_Type, &addresses, &PyType_Type, &tiled, &PyType_Type, &paged)) return nullptr;
+  PyObject *addresses, *tiled, *paged, *error;
+  if (!PyArg_ParseTuple(args, "O!O!O!O!", &PyTuple_Type, &addresses, &PyType_Type, &tiled, &PyType_Type, &paged, &PyType_Type,
+                        &error))
+    return nullptr;
   constexpr Py_ssize_t kEntries = sizeof(Library) / sizeof(void*);
   if (PyTuple_GET_SIZE(addresses) != kEntries) {
     PyErr_SetString(PyExc_ValueError, "wrong number of entry points");
@@ -677,6 +693,8 @@ PyObject* bind(PyObject*, PyObject* args) {
   std::memcpy(&g_lib, entry, sizeof(g_lib));
   Py_INCREF(tiled);
   Py_INCREF(paged);
+  Py_INCREF(error);
+  g_error = error;
   g_tiled = reinterpret_cast<PyTypeObject*>(tiled);
   g_paged = reinterpret_cast<PyTypeObject*>(paged);
   Py_RETURN_NONE;

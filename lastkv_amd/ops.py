@@ -174,8 +174,9 @@ def _bind_host() -> bool:
     if _host is None:
         raise _lib.LastKVNativeError("_host.so is not built; run `python -m lastkv_amd.build`")
     names = ("lkv_decode_attn", "lkv_decode_workspace_bytes", "lkv_prefill_attn", "lkv_prefill_workspace_bytes",
-             "lkv_qkv_epilogue", "lkv_rmsnorm", "lkv_silu_mul")
-    _host.bind(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), TiledKV, PagedKV)
+             "lkv_qkv_epilogue", "lkv_rmsnorm", "lkv_silu_mul", "lkv_last_error")
+    _host.bind(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), TiledKV, PagedKV,
+               _lib.LastKVNativeError)
     _host_bound = True
     return True
 

@@ -220,3 +220,37 @@ def test_refused_calls_raise_as_before(bad):
             ops.silu_mul(q, q[:, :4])
         else:
             ops.rmsnorm(_randn(1, 4, 65)[:, 1:], _randn(1, 64), 1e-5)
+
+
+@pytest.mark.parametrize("op", ["rmsnorm", "rmsnorm_in_place", "silu_in_place", "decode", "prefill", "epilogue"])
+def test_a_reported_hip_error_raises_and_issues_the_call_once(op):
+    """A HIP error that an earlier call left on the thread is reported by the next launch, whose kernel runs all
+    the same: the call raises, as the Python bodies do, and its work is not issued a second time (in-place
+    results would take it twice)."""
+
+    x, r, w = _randn(1, 3, 64), _randn(2, 3, 64), _randn(3, 64)
+    seg, q = _segments("tiled"), _randn(11, B, HQ, D)
+    rows = [_randn(s, B, 1, n * D) for s, n in ((13, HQ), (14, HKV), (15, HKV))] + [_randn(s, 1, 1, D) for s in (16, 17)]
+    ring = _tiled(18, B, 3)
+    calls = {
+        "rmsnorm": lambda: ops.rmsnorm(x, w, 1e-5, residual=r),
+        "rmsnorm_in_place": lambda: ops.rmsnorm(x, w, 1e-5, out=x),
+        "silu_in_place": lambda: ops.silu_mul(x, r, out=x),
+        "decode": lambda: ops.decode_attention(q, num_splits=1, **seg),
+        "prefill": lambda: ops.prefill_attention(q[:, None], **seg),
+        "epilogue": lambda: ops.qkv_epilogue(*rows, num_q_heads=HQ, num_kv_heads=HKV, q_norm_weight=None, k_norm_weight=None,
+                                             eps=1e-5, positions=3, ring=ring),
+    }
+    once = [x.clone(), r.clone()]
+    if op == "rmsnorm":
+        ops.rmsnorm(once[0], w, 1e-5, residual=once[1])
+    elif op == "rmsnorm_in_place":
+        ops.rmsnorm(once[0], w, 1e-5, out=once[0])
+    elif op == "silu_in_place":
+        ops.silu_mul(once[0], once[1], out=once[0])
+    torch.cuda.synchronize()
+    assert _lib.load().hipSetDevice(9999) != 0  # (resolved from the HIP runtime the library is linked with)
+    with pytest.raises(_lib.LastKVNativeError, match="status 4"):
+        calls[op]()
+    torch.cuda.synchronize()
+    assert torch.equal(x, once[0]) and torch.equal(r, once[1])
