@@ -253,7 +253,7 @@ int32_t plan_short_rows(const lkv_prefill_args* a, const SegParams& seg, int32_t
   plan.items = class_n > 0 ? int64_t{class_n} * a->num_kv_heads * p.splits : 0;
   plan.vscale = a->older_vscale_mode == 1;
   plan.nt = use_nontemporal(0, pairs * tokens * kHeadDim * 2 * 2);
-  p.interleave = plan.nt && seg.o_tab == nullptr && seg.l_tab == nullptr;
+  p.interleave = seg.o_tab == nullptr && seg.l_tab == nullptr;
   // the instance holds the class's widest sequence: 16, 32 or 64 columns
   const int64_t cols = std::min<int64_t>(col_hi, static_cast<int64_t>(group) * p.L);
   plan.cg = cols <= 16 ? 1 : cols <= 32 ? 2 : 4;
@@ -349,8 +349,7 @@ int32_t run_decode(const lkv_decode_args* a, void* ws, int64_t ws_bytes, hipStre
   p.splits = a->num_splits;
   p.scale_log2 = a->sm_scale * kLog2e;
   const int64_t kv_bytes = static_cast<int64_t>(a->batch) * a->num_kv_heads * call_key_tokens(a) * kHeadDim * 2 * 2;
-  // (by size, whatever the hint: results do not depend on it)
-  p.interleave = use_nontemporal(0, kv_bytes) && p.seg.o_tab == nullptr && p.seg.l_tab == nullptr;
+  p.interleave = p.seg.o_tab == nullptr && p.seg.l_tab == nullptr;
   // groups above 16 query heads per kv head take the multi-column instances (columns = heads)
   const int cg = group <= 16 ? 0 : group <= 32 ? 2 : 4;
   return launch_decode(p, dim3(a->num_splits, a->num_kv_heads, a->batch), a->older_vscale_mode == 1,

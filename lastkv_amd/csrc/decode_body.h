@@ -9,6 +9,7 @@ namespace lkv {
 
 constexpr int kDecodeWaves = 4;
 constexpr float kDecodeNegInf = -__builtin_inff();
+constexpr int kInterleaveBlocks = 3072;  // (96K keys; see decode_split_body)
 constexpr float kLazyRaise = 8.f;  // exp2 units a block maximum may exceed m before m is raised
 
 struct DecodeParams {
@@ -34,7 +35,7 @@ struct DecodeParams {
   const int32_t* cu;
   int32_t rows, col_lo, col_hi;
   int32_t dyn_splits, cus, lmax;
-  int32_t interleave;  // key splits take interleaved blocks (large tiled calls) instead of contiguous ranges
+  int32_t interleave;  // tiled caches: sequences of more than kInterleaveBlocks key blocks interleave their splits
 };
 
 // Query tokens of sequence b (kMulti calls) and the flattened row of its token 0 (the q / out / lse
@@ -302,17 +303,20 @@ __device__ __attribute__((always_inline)) inline void decode_split_body(const De
 
   const SeqView sv = make_seq_view(p.seg, b, kvh);
   const int nbt = sv.nb0 + (sv.n1 > 0 ? (sv.lead + sv.n1 + kBlockTokens - 1) / kBlockTokens : 0);
-  // Large calls over tiled caches interleave their splits: wave w of split s takes blocks s * kStride + w, + S * kStride, ...,
+  // Long sequences in tiled caches interleave their splits: wave w of split s takes blocks s * kStride + w, + S * kStride, ...,
   // so that the workgroups of one (sequence, kv head) walk one window of its K and V together: fewer DRAM
-  // pages are open at once than with a contiguous range per split (128K keys: 4 sequences 330 -> 318 us, 2
-  // sequences 190 -> 168, one 100 -> 87).  Below 384 MiB of K/V, which the last-level cache partly holds,
-  // ranges were up to 4 % faster (7 sequences at 16K, 4 kv heads: 47.4 against 49.2 us), as they were for
-  // paged segments (9 sequences at 16K: 104.6 against 107.3), whose page ids would then come from another
-  // cache line of the table for every block.
+  // pages are open at once than with a contiguous range per split.  At 128K keys, us with ranges and
+  // interleaved: 1, 2 and 4 sequences of 8 kv heads 95.2 / 84.0, 175 / 166, 345 / 325, of 4 heads 50.6 / 48.9,
+  // 96.8 / 86.7, 178 / 166, of 12 heads 129 / 124, 253 / 247, 492 / 482.  At 64K the two are within 2 % (4
+  // sequences of 8 heads 164 / 167.5), at 8K ranges are ahead (16 sequences 86.5 / 91.6).  The line is a
+  // sequence's own key count, so that its bits do not change with the call's other sequences or the size
+  // of its cache.  Paged segments keep ranges: a block's page id would come from another cache line of the table
+  // than the wave's last (9 sequences at 16K: 104.6 with ranges, 107.3 interleaved).
   const int bps = (nbt + S - 1) / S;
-  const int step = p.interleave ? S * kStride : kStride;
-  const int blk_begin = p.interleave ? split * kStride : split * bps;
-  const int blk_end = p.interleave ? nbt : min(blk_begin + bps, nbt);
+  const bool interleave = p.interleave && nbt > kInterleaveBlocks;
+  const int step = interleave ? S * kStride : kStride;
+  const int blk_begin = interleave ? split * kStride : split * bps;
+  const int blk_end = interleave ? nbt : min(blk_begin + bps, nbt);
 
   const int cols = kMulti ? G * Lq : G;
   uint4 qf[CG][4];

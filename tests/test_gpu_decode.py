@@ -416,3 +416,41 @@ def test_decode_lazy_rescale_threshold_regimes(name):
     out = ops.prefill_attention(_t(q2), older=cache, older_len=blocks * 32, causal=True, sm_scale=sm)
     want2, _ = A.attention(q2.transpose(0, 2, 1, 3), k, v, scale=sm)
     _close(out, bf16.round_bf16(want2.transpose(0, 2, 1, 3).astype(np.float32)), f"lazy {name} short prefill")
+
+
+@pytest.mark.parametrize("tokens", [1, 3])
+def test_fixed_splits_give_a_sequence_the_same_bits_in_any_call(tokens):
+    """With a fixed split count a sequence's result does not depend on the call around it: alone, beside enough
+    other sequences that the call's K/V pass 384 MiB, and with its lengths on the device in caches of twice its
+    size.  (8 kv heads, 8K keys: 32 MiB a sequence; a sequence of 100K keys interleaves its splits.)"""
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    B, H, T, splits = 13, 8, 8192, 3
+    rnd = lambda *shape: torch.randn(shape, generator=g, device=DEV, dtype=torch.bfloat16)  # noqa: E731
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+
+    def call(q, cache, n, slots):
+        if tokens == 1:
+            return ops.decode_attention(q[:, 0], older=cache, older_len=n, older_slot=slots, num_splits=splits)
+        return ops.prefill_attention(q, older=cache, older_len=n, older_slot=slots, num_splits=splits)
+
+    q = rnd(B, tokens, H, 128)
+    cache = ops.TiledKV(rnd(B, H, T // 32, 4096), rnd(B, H, T // 32, 4096))
+    together = call(q, cache, T, None)
+    roomy = ops.TiledKV.zeros(4, H, 4 * T, DEV)
+    for b in (0, 7):
+        assert torch.equal(call(q[b:b + 1], cache, T, i32(b))[0], together[b])
+        roomy.k[1, :, :T // 32], roomy.v[1, :, :T // 32] = cache.k[b], cache.v[b]
+        got = call(q[b:b + 1].expand(4, -1, -1, -1).contiguous(), roomy, i32(T, T, T, T), i32(0, 1, 2, 3))
+        assert torch.equal(got[1], together[b])
+    n = 100_000  # one long sequence beside short ones
+    long = ops.TiledKV(rnd(1, H, n // 32, 4096), rnd(1, H, n // 32, 4096))
+    alone = call(q[:1], long, n, None)
+    beside = call(q[:1].expand(3, -1, -1, -1).contiguous(), long, i32(77, n, 4000), i32(0, 0, 0))
+    assert torch.equal(beside[1], alone[0])
+    # (and it is the attention over its keys: its first kv head against the fp32 product)
+    k, v = ops.unpack_kv(long, 0, n)
+    s = q[0, :, 0].float() @ k[0, 0].float().t().contiguous() / 128 ** 0.5
+    want = (torch.softmax(s, -1) @ v[0, 0].float()).bfloat16()
+    got = alone[0].view(tokens, H, 128)[:, 0] if tokens > 1 else alone[0, :1]
+    _close(got, want.float().cpu().numpy(), f"100K keys, {tokens} tokens")
