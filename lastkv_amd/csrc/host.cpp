@@ -62,9 +62,11 @@ bool plain_mode() {
   return !c10::impl::TorchDispatchModeTLS::any_modes_set() && !at::impl::torch_function_mode_enabled();
 }
 
+// As Tensor.data_ptr() in Python: a copy-on-write tensor gets memory of its own first.  (Inputs too: one call may
+// write a tensor that another of its arguments views, and both must then name the same memory.)
 template <class T = void>
 T* ptr(const at::Tensor& t) {
-  return static_cast<T*>(const_cast<void*>(t.const_data_ptr()));
+  return static_cast<T*>(t.mutable_data_ptr());
 }
 
 bool as_int(PyObject* o, int64_t& v) {

@@ -254,3 +254,44 @@ def test_a_reported_hip_error_raises_and_issues_the_call_once(op):
         calls[op]()
     torch.cuda.synchronize()
     assert torch.equal(x, once[0]) and torch.equal(r, once[1])
+
+
+@pytest.mark.parametrize("what", ["norm_out", "residual", "silu_out", "decode", "prefill", "epilogue"])
+def test_outputs_detach_copy_on_write_tensors(what):
+    """A lazily cloned tensor shares its storage until one of the two is written: what a call writes (outputs, LSE,
+    residual, caches, workspace) is the written tensor's own memory."""
+
+    def lazy(t):
+        return t, t.clone(), torch._lazy_clone(t)
+
+    x, w = _randn(1, 3, 64), _randn(3, 64)
+    q, seg = _randn(11, B, HQ, D), _segments("tiled")
+    shared = []
+
+    def out(t):
+        shared.append(lazy(t))
+        return shared[-1][2]
+
+    if what == "norm_out":
+        ops.rmsnorm(x, w, 1e-5, out=out(_randn(2, 3, 64)))
+    elif what == "residual":
+        ops.rmsnorm(x, w, 1e-5, residual=out(_randn(2, 3, 64)))
+    elif what == "silu_out":
+        ops.silu_mul(x, x, out=out(_randn(2, 3, 64)))
+    elif what in ("decode", "prefill"):
+        ws = torch.zeros(1 << 20, dtype=torch.uint8, device=DEV)
+        if what == "decode":
+            ops.decode_attention(q, num_splits=2, out=out(_randn(2, B, HQ, D)), lse=out(torch.zeros(B, HQ, device=DEV)),
+                                 workspace=out(ws), **seg)
+        else:
+            ops.prefill_attention(_randn(12, B, 40, HQ, D), out=out(_randn(2, B, 40, HQ, D)),
+                                  lse=out(torch.zeros(B, 40, HQ, device=DEV)),
+                                  workspace=out(torch.zeros(4 << 20, dtype=torch.uint8, device=DEV)), **seg)
+    else:
+        ring, deep = (ops.TiledKV(*(out(t) for t in (kv.k, kv.v))) for kv in (_tiled(16, B, 3), _tiled(18, B, 8)))
+        ops.qkv_epilogue(*(_randn(s, B, 20, n * D) for s, n in ((13, HQ), (14, HKV), (15, HKV))),
+                         *(_randn(s, 1, 20, D) for s in (16, 17)), num_q_heads=HQ, num_kv_heads=HKV, q_norm_weight=None,
+                         k_norm_weight=None, eps=1e-5, positions=3, ring=ring, deep=deep, q_out=out(_randn(2, B, 20, HQ, D)))
+    torch.cuda.synchronize()
+    for original, before, written in shared:
+        assert torch.equal(original, before) and not torch.equal(written, before)
