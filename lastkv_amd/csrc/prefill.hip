@@ -220,9 +220,9 @@ struct RowState {
 
 // Raises each row's reference to its maximum over this block (lm = lane maxima) and rescales O
 // and the row sums by 2^(mc_old - mc_new).  Runs for the first block and in a wave-uniform branch
-// taken whenever some P reached 2^9.  unset: mc of a row that has seen no key (with kUnset its first
-// key's P overflows, so that the branch gives the row its reference).
-constexpr float kUnset = -1e30f;
+// taken whenever some P reached 2^9.  unset: mc of a row that has seen no score above -inf (with kUnset, the
+// lowest finite float, the P of its first finite score overflows, so that the branch gives the row its reference).
+constexpr float kUnset = -3.40282346638528859812e38f;
 __device__ inline void raise_rows(RowState& rs, float lm, float c, f32x4 (&o)[8], f32x4& ol, float unset = 0.f) {
   const float bm = wave_max_across_rows(lm);
   const bool up = bm > rs.m;  // m = -inf: true for the first finite maximum
@@ -435,10 +435,14 @@ constexpr int kTileRing = 4;       // LDS block buffers of the tile kernel
 constexpr int kTileBuf = 1024;     // uint4 per block buffer (16 KiB)
 
 // The key splits a tile of nbt key blocks, nb0 of them older ones, takes of S offered: 4-wave tiles as many
-// as leave each kMinSplitBlocks, wherever they start (a row that sees no key in its split's first block
-// takes its reference from the first block it sees).  Wider tiles, whose loop does not test for such rows,
-// and calls with an older segment of 1 to kMinOlderBlocks - 1 blocks (no chunk of 256 tokens or more leaves
-// one so short): as many equal ones as start inside the older segment, whose blocks every row sees.
+// as leave each kMinSplitBlocks, wherever they start (the keys a row sees are a prefix of [older | local]: a row
+// that sees none in its split's first block sees none in the split, whose state for it is empty).  Wider tiles
+// as many equal ones as start inside the older segment, whose blocks every row sees (they split only grids of
+// at most half the CUs; starts in the local segment were not measured for them).  So do calls with an older
+// segment of 1 to kMinOlderBlocks - 1 blocks: they give the bits of the unsplit call where no equal split starts
+// inside it, which callers with a short older segment rely on; with splits anywhere, 512 tokens over 70
+// older and 2048 local keys (one sequence, 32 query and 8 kv heads) would take 42 us instead of 53, 64 tokens
+// 29 instead of 52, and calls of less than 600 keys in all the same 16-22.
 constexpr int kMinSplitBlocks = 4, kMinOlderBlocks = 8;
 
 __host__ __device__ inline int effective_splits(int S, int nbt, int nb0, int waves) {
@@ -471,7 +475,7 @@ template <int NW, int CG, bool kPaged, bool kWide = false, int KS = 1>
 __device__ __attribute__((always_inline)) inline void prefill_tile(const PrefillParams& p, const int b, const int kvh,
                                                                    const int tile, const int split, uint4* lds) {
   constexpr bool kSplitP = NW == 2 || kWide;
-  constexpr bool kAnyStart = NW == 4 && !kWide;  // key splits may start where some rows see no key
+  constexpr bool kAnyStart = NW == 4 && !kWide;  // key splits may start in the local segment
   constexpr float kUnsetMc = kAnyStart ? kUnset : 0.f;
   constexpr int kStages = 2;  // register stage sets (global loads run kStages steps ahead of their LDS store)
   constexpr int kDist = 2;    // step i stores block i + kDist into the LDS ring
@@ -628,10 +632,10 @@ __device__ __attribute__((always_inline)) inline void prefill_tile(const Prefill
         sc[cg][1] = mfma_bf16(k1, qf[cg][kb], sc[cg][1]);
       }
     }
-    // Block 0 sets every row's reference to its exact maximum (a row that sees any key sees one
-    // in block 0: visible keys are a prefix of [older | local]; a key split may start past a row's last
-    // key of its first block, and the row's reference kUnset then sends the wave through the rescale
-    // branch at the row's first key: the few blocks at the causal edge).  Inside the loop the only rescale
+    // Block 0 sets every row's reference to its exact maximum (a row that sees any key of the split sees one
+    // in its block 0: visible keys are a prefix of [older | local]).  A row whose scores there are all
+    // -inf (sums beyond fp32) gets kUnset: its first finite score then overflows P and takes the wave through
+    // the rescale branch, where a reference of 0 would lose scores below -24.  Inside the loop the only rescale
     // test is then the packed-probability overflow check, so the compiler keeps the QK^T MFMAs of
     // block i + 1 and the probabilities of block i in one scheduling region and interleaves them.
     {

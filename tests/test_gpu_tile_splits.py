@@ -225,3 +225,23 @@ def test_a_nan_key_reaches_every_row_that_sees_it(B, L, T0, tile_waves):
         for splits in (0, 1):
             got = ops.prefill_attention(q, causal=True, tile_waves=tile_waves, num_splits=splits, **seg)
             assert torch.equal(torch.isnan(got), want), f"key {at}, num_splits {splits}"
+
+
+def test_a_split_whose_first_scores_overflow_keeps_its_later_keys():
+    """4-wave tiles with key splits, every key range's first block at scores of -infinity (their fp32 sums
+    overflow) and all later keys at one finite score of -1.02e33: the output is the mean of V over the later keys, as
+    no finite score is lower than the reference of a row that has none yet.  (Every split holds as many keys: in an
+    fp32 LSE of this magnitude the logarithm of their number is lost.)"""
+
+    B, Hkv, G, L, n = 1, 2, 2, 64, 1024  # 32 blocks: four splits of two halves of 4
+    q = torch.full((B, L, Hkv * G, 128), 8.0, dtype=torch.bfloat16, device=DEV)
+    k = torch.full((B, Hkv, n, 128), -1e30, dtype=torch.bfloat16, device=DEV)
+    v = torch.randn((B, Hkv, n, 128), generator=torch.Generator(device=DEV).manual_seed(2), device=DEV).bfloat16()
+    first = (torch.arange(n, device=DEV) // 32) % 4 == 0
+    k[:, :, first] = -3e38
+    cache = ops.TiledKV.zeros(B, Hkv, n, DEV)
+    ops.pack_kv(k, v, cache)
+    # sm_scale log2(e) = 1: the scaled scores are the sums themselves
+    got = ops.prefill_attention(q, local=cache, local_len=n, causal=False, sm_scale=float(np.log(2.0)), tile_waves=4)[0].double()
+    want = torch.stack([v[0, h // G, ~first].double().mean(0) for h in range(Hkv * G)]).bfloat16().double()[None]
+    assert float((got - want).norm() / want.expand_as(got).norm()) <= REL_L2
