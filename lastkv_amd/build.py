@@ -85,13 +85,13 @@ def build(verbose: bool = False) -> pathlib.Path:
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources) + 1)) as pool:
         host = pool.submit(_build_host)
         objs = list(pool.map(lambda s: _compile(s, verbose), sources))
-        host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    host.result()  # (after the link: the library is complete without the launch module)
     return LIB_PATH
 
 

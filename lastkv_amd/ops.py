@@ -6,7 +6,8 @@ the CPU; a missing library raises ``LastKVNativeError``.
 
 The hot ops (attention, epilogue, RMSNorm, SwiGLU) first hand their arguments to ``_host``
 (csrc/host.cpp), which makes the same checks and the same call natively for the common argument
-forms; where it answers None, the Python body below it checks, reports and calls as it always did.
+forms; where it answers None, or is not built, the Python body below it checks, reports and makes the
+call.
 """
 
 from __future__ import annotations
@@ -22,7 +23,7 @@ from . import _lib
 
 try:
     from . import _host
-except ImportError:  # not built: _bind_host raises at the first call
+except ImportError:  # not built (or for another torch): the Python bodies make every call
     _host = None
 
 HEAD_DIM = 128
@@ -163,16 +164,16 @@ _host_bound = False
 
 
 def _bind_host() -> bool:
-    """Give ``_host`` the library's entry points (once per process); False when the library is missing
-    (the Python bodies then raise after their own checks)."""
+    """Give ``_host`` the library's entry points (once per process); False without ``_host`` and when the
+    library is missing (the Python bodies then raise after their own checks)."""
 
     global _host_bound
+    if _host is None:
+        return False
     try:
         lib = _lib.load()
     except _lib.LastKVNativeError:
         return False
-    if _host is None:
-        raise _lib.LastKVNativeError("_host.so is not built; run `python -m lastkv_amd.build`")
     names = ("lkv_decode_attn", "lkv_decode_workspace_bytes", "lkv_prefill_attn", "lkv_prefill_workspace_bytes",
              "lkv_qkv_epilogue", "lkv_rmsnorm", "lkv_silu_mul", "lkv_last_error")
     _host.bind(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), TiledKV, PagedKV,
