@@ -353,6 +353,14 @@ PyObject* decode_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
   });
 }
 
+// A buffer export, given back at the end of its scope.
+struct Buffer {
+  Py_buffer view{};
+  ~Buffer() {
+    if (view.obj != nullptr) PyBuffer_Release(&view);
+  }
+};
+
 // (q, older, older_len, older_slot, vscale, local, local_len, local_start, local_slot, older_table, local_table,
 //  local_ring_blocks, causal, sm_scale, out, lse, workspace, tile_waves, out_scale, cu_seqlens_q, max_seqlen_q,
 //  num_splits, cu_seqlens_q_host)
@@ -413,41 +421,33 @@ PyObject* prefill_attention(PyObject*, PyObject* const* v, Py_ssize_t n) {
     a.out_stride_b = ragged ? out.stride(0) * L : out.stride(0);
     a.out_stride_t = ragged ? out.stride(0) : out.stride(1);
     a.lse = lse ? ptr<float>(*lse) : nullptr;
-    Py_buffer host;
-    host.obj = nullptr;
+    Buffer host;
     if (ragged && v[22] != Py_None) {  // B + 1 non-decreasing int32 offsets from 0
-      if (!PyObject_CheckBuffer(v[22]) || PyObject_GetBuffer(v[22], &host, PyBUF_FORMAT | PyBUF_ND | PyBUF_C_CONTIGUOUS) != 0) {
+      if (!PyObject_CheckBuffer(v[22]) ||
+          PyObject_GetBuffer(v[22], &host.view, PyBUF_FORMAT | PyBUF_ND | PyBUF_C_CONTIGUOUS) != 0) {
         PyErr_Clear();
         return not_handled();
       }
-      const int32_t* cu = static_cast<const int32_t*>(host.buf);
-      bool ok = host.ndim == 1 && host.itemsize == 4 && host.format != nullptr && std::strcmp(host.format, "i") == 0 &&
-                host.len == 4 * (B + 1) && cu[0] == 0;
+      const Py_buffer& h = host.view;
+      const int32_t* cu = static_cast<const int32_t*>(h.buf);
+      bool ok = h.ndim == 1 && h.itemsize == 4 && h.format != nullptr && std::strcmp(h.format, "i") == 0 &&
+                h.len == 4 * (B + 1) && cu[0] == 0;
       for (int64_t b = 0; ok && b < B; ++b) ok = cu[b + 1] >= cu[b];
-      if (!ok) {
-        PyBuffer_Release(&host);
-        return not_handled();
-      }
+      if (!ok) return not_handled();
       a.cu_seqlens_q_host = cu;
     }
     at::Tensor ws;
-    bool ok = true;
     if (v[16] != Py_None) {
       const at::Tensor* w = tensor(v[16]);
-      ok = w != nullptr && w->device() == dev && w->is_contiguous();
-      if (ok) ws = *w;
+      if (w == nullptr || w->device() != dev || !w->is_contiguous()) return not_handled();
+      ws = *w;
     } else {
       ws = new_bytes(std::max<int64_t>(16, g_lib.prefill_workspace_bytes(&a)), dev);
     }
-    PyObject* done = nullptr;
-    if (ok) {
-      a.workspace = ptr(ws);
-      a.workspace_bytes = static_cast<int64_t>(ws.nbytes());
-      const lkv_stream_t s = stream_of(*q);
-      done = issue("lkv_prefill_attn", v[14], out, [&] { return g_lib.prefill_attn(&a, s); });
-    }
-    if (host.obj != nullptr) PyBuffer_Release(&host);
-    return ok ? done : not_handled();
+    a.workspace = ptr(ws);
+    a.workspace_bytes = static_cast<int64_t>(ws.nbytes());
+    const lkv_stream_t s = stream_of(*q);
+    return issue("lkv_prefill_attn", v[14], out, [&] { return g_lib.prefill_attn(&a, s); });
   });
 }
 

@@ -3,6 +3,8 @@ forms both take: same bits, same refusals."""
 
 from __future__ import annotations
 
+import array
+
 import numpy as np
 import pytest
 import torch
@@ -295,3 +297,24 @@ def test_outputs_detach_copy_on_write_tensors(what):
     torch.cuda.synchronize()
     for original, before, written in shared:
         assert torch.equal(original, before) and not torch.equal(written, before)
+
+
+def test_a_failed_allocation_gives_the_host_offsets_back():
+    """cu_seqlens_q_host is read through the buffer protocol: a call whose workspace cannot be allocated raises and
+    keeps no hold of the caller's array (an array.array that is exported cannot grow)."""
+
+    cu = array.array("i", [0, 40, 41, 43])
+    q = _randn(12, 43, HQ, D)
+    # (1.6 GB of workspace: the table could name that many blocks; more than any hole the allocator still has)
+    table = (torch.arange(B * 32768, dtype=torch.int32, device=DEV) % 64).view(B, 32768)
+    seg = dict(older=_paged(5, 64), older_table=table, older_len=_i32(200, 31, 256))
+    out, cu_dev = torch.empty_like(q), _i32(*cu)
+    ops.prefill_attention(q, out=out, cu_seqlens_q=cu_dev, max_seqlen_q=40, cu_seqlens_q_host=cu, **seg)
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(1e-6)
+    try:
+        with pytest.raises(torch.cuda.OutOfMemoryError):
+            ops.prefill_attention(q, out=out, cu_seqlens_q=cu_dev, max_seqlen_q=40, cu_seqlens_q_host=cu, **seg)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    cu.append(43)
