@@ -301,6 +301,19 @@ int64_t lkv_prefill_workspace_bytes(const lkv_prefill_args *args);
  * their own scratch); for callers that size one workspace for many calls. */
 int64_t lkv_prefill_workspace_min_bytes(const lkv_prefill_args *args);
 
+/* How lkv_prefill_attn runs the sequences above 64 query rows per kv head of these args (their workspace
+ * included); all 0 when no tile kernel runs.  No launch is made and no pointer but cu_seqlens_q_host is read.
+ * For tests and tuning; no counterpart in the reference. */
+typedef struct lkv_prefill_plan_info {
+  int32_t tile_waves;        /* waves of one key range's query tile: 2, 4 or 8 */
+  int32_t tile_splits;       /* key splits whose states are merged through the workspace (1: none) */
+  int32_t key_halves;        /* 1: each workgroup holds two key ranges and merges them itself */
+  int32_t rows_beside_tiles; /* 1: the sequences of 1-16 query rows per kv head share the tiles' launch */
+  int64_t tile_workgroups;
+} lkv_prefill_plan_info;
+
+int32_t lkv_prefill_plan(const lkv_prefill_args *args, lkv_prefill_plan_info *info);
+
 int32_t lkv_prefill_attn(const lkv_prefill_args *args, lkv_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------

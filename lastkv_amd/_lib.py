@@ -137,6 +137,18 @@ class PrefillArgs(ctypes.Structure):
     ]
 
 
+class PrefillPlanInfo(ctypes.Structure):
+    """lkv_prefill_plan_info."""
+
+    _fields_ = [
+        ("tile_waves", c_i32),
+        ("tile_splits", c_i32),
+        ("key_halves", c_i32),
+        ("rows_beside_tiles", c_i32),
+        ("tile_workgroups", c_i64),
+    ]
+
+
 class AppendArgs(ctypes.Structure):
     """Mirror of ``lkv_append_args``."""
 
@@ -328,6 +340,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "lkv_decode_attn_noalloc": (c_i32, [ctypes.POINTER(DecodeArgs), c_ptr]),
     "lkv_prefill_workspace_bytes": (c_i64, [ctypes.POINTER(PrefillArgs)]),
     "lkv_prefill_workspace_min_bytes": (c_i64, [ctypes.POINTER(PrefillArgs)]),
+    "lkv_prefill_plan": (c_i32, [ctypes.POINTER(PrefillArgs), ctypes.POINTER(PrefillPlanInfo)]),
     "lkv_prefill_attn": (c_i32, [ctypes.POINTER(PrefillArgs), c_ptr]),
     "lkv_merge_states": (c_i32, [ctypes.POINTER(MergeArgs), c_ptr]),
     "lkv_append_paged": (c_i32, [ctypes.POINTER(AppendArgs), c_ptr]),

@@ -1324,7 +1324,10 @@ void launch_wide(int waves, bool paged, int pair_wgs, const lkv::PrefillParams& 
     prefill_wide_kernel<2, 2, 1, false><<<grid, 2 * 64, 0, s>>>(p);
 }
 
-extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stream) {
+namespace {
+
+// Argument checks of lkv_prefill_attn and lkv_prefill_plan (no device calls but the CU count); fills seg.
+int32_t check_prefill_args(const lkv_prefill_args* a, lkv::SegParams& seg) {
   using namespace lkv;
   LKV_REQUIRE(a != nullptr, "null args");
   LKV_REQUIRE(a->struct_size == static_cast<int32_t>(sizeof(lkv_prefill_args)),
@@ -1355,12 +1358,9 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
                   a->local_len_const >= a->tokens,
               "causal calls need local_len >= tokens (the queries' own keys end the local segment), got %d < %d",
               a->local_len_const, a->tokens);
-  PrefillParams p;
-  if (const int32_t st = fill_segments(a, p.seg)) return st;
+  if (const int32_t st = fill_segments(a, seg)) return st;
   LKV_REQUIRE(a->batch <= 65535 && a->num_kv_heads <= 65535, "batch and num_kv_heads must be <= 65535");
   if (a->batch == 0 || a->tokens == 0) return LKV_OK;
-  // query tokens per sequence (ragged: an upper bound)
-  const int64_t seq_tokens = ragged ? std::min(a->max_seqlen_q, a->tokens) : a->tokens;
   const int64_t vblocks = v16_blocks(a);
   const int64_t need = min_workspace_bytes(a);
   LKV_REQUIRE(vblocks * kBlockElems * 2 < (1LL << 31), "too many key blocks per sequence");
@@ -1370,54 +1370,137 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
               static_cast<long long>(need), static_cast<long long>(lkv_prefill_workspace_bytes(a)),
               static_cast<long long>(a->workspace_bytes));
   LKV_REQUIRE((reinterpret_cast<uintptr_t>(a->workspace) & 15) == 0, "workspace must be 16-byte aligned");
-  hipStream_t s = as_stream(stream);
+  return LKV_OK;
+}
+
+// What a call with work to do launches, from its checked arguments.
+struct CallPlan {
+  TilePlan tile;
+  HostPlan host;
+  int64_t vblocks, v16_bytes;  // key blocks per (sequence, kv head) in the workspace, and their region
+  bool short_on_decode;        // sequences of at most 64 query rows per kv head run on the decode kernel
+  bool runs_tiles;
+  int splits;                  // key splits of the tile grid (1: none)
+  bool halves;                 // its workgroups take two key halves each
+  bool mixed;                  // the 1-16 column class runs in one launch with the tiles, as rows16 says
+  lkv::ShortRowsPlan rows16;
+};
+
+int32_t plan_call(const lkv_prefill_args* a, const lkv::SegParams& seg, CallPlan& c) {
+  using namespace lkv;
+  const bool ragged = a->cu_seqlens_q != nullptr;
+  const int group = a->num_q_heads / a->num_kv_heads;
+  const int64_t seq_tokens = ragged ? std::min(a->max_seqlen_q, a->tokens) : a->tokens;
+  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  c.vblocks = v16_blocks(a);
+  c.v16_bytes = v16_region_bytes(a, c.vblocks);
+  c.tile = tile_plan(a);
+  c.host = host_plan(a, group);
   // Sequences of at most 64 query rows per kv head (e.g. decode tokens, or up to 16 tokens of a GQA
   // group of 4) read every key once on the decode kernel (one score column per (token, head))
   // instead of converting V to fp16 and running 2-wave tiles; tile_waves 4 or 8 keep a uniform call
   // on the tile kernel.  A ragged call runs its sequences of 1-16, 17-32 and 33-64 columns on the
   // decode instance of that width (one launch per class present) and the longer ones on the tile
   // kernel, also with tile_waves 4 or 8 unless all of its sequences are short.
-  const int64_t max_cols = seq_tokens * group;
-  const bool short_on_decode = a->tile_waves == 0 || ragged_short_on_decode(a);
-  const TilePlan plan = tile_plan(a);
+  c.short_on_decode = a->tile_waves == 0 || ragged_short_on_decode(a);
+  c.runs_tiles = !c.short_on_decode || (seq_tokens * group > 64 && (!c.host.known || c.host.any_tile));
   // key splits: as many as the workspace holds the states of (1 without room)
-  int splits = plan.splits;
-  const int64_t v16_bytes = v16_region_bytes(a, vblocks);
-  while (splits > 1 && v16_bytes + tile_split_bytes(a, plan, splits) > a->workspace_bytes) --splits;
-  if (vblocks == 0) splits = 1;
-  ShortRowsPlan rows16;  // the 1-16 column class, when it runs in one launch with the tiles
-  bool mixed = false;
-  if (short_on_decode) {
-    // (with the host copy of a ragged call's offsets: only the classes that hold a sequence)
-    const HostPlan hp = host_plan(a, group);
-    const int32_t bounds[4] = {0, 16, 32, 64};
-    // A step whose class of 1-16 columns and whose tiles both hold sequences runs the two in one launch
-    // (mixed_step_kernel), when the host knows the class's count (its grid then holds exactly its work
-    // items), the split counts are the library's and the class's split states fit behind the tiles' (in
-    // the launch of their own they are the workspace's first bytes, which the pre-pass writes here).
-    if (hp.known && hp.any_tile && hp.class_n[0] > 0 && plan.waves == 4 && a->num_splits == 0 && vblocks > 0) {
-      const int64_t used = (v16_bytes + tile_split_bytes(a, plan, splits) + 15) / 16 * 16;
-      if (const int32_t st = plan_short_rows(a, p.seg, group, 0, 16, hp.class_n[0], nullptr, int64_t{1} << 62, rows16)) return st;
-      const int64_t room = std::max<int64_t>(0, a->workspace_bytes - used);
-      mixed = !rows16.empty && (rows16.p.splits == 1 || rows16.state_bytes <= room);
-      if (mixed && rows16.p.splits > 1) {
-        if (const int32_t st = plan_short_rows(a, p.seg, group, 0, 16, hp.class_n[0],
-                                               static_cast<uint8_t*>(a->workspace) + used, room, rows16))
-          return st;
-      }
-    }
-    for (int c = 0; c < 3; ++c) {
-      if (c == 0 && mixed) continue;
-      if (max_cols <= bounds[c]) break;
-      // a uniform call is one class: the one its width falls in
-      if (!ragged && max_cols > bounds[c + 1]) continue;
-      if (hp.known && hp.class_n[c] == 0) continue;
-      if (const int32_t st = prefill_on_decode_kernel(a, p.seg, group, bounds[c], bounds[c + 1],
-                                                      hp.known ? hp.class_n[c] : -1, s))
+  c.splits = c.tile.splits;
+  while (c.splits > 1 && c.v16_bytes + tile_split_bytes(a, c.tile, c.splits) > a->workspace_bytes) --c.splits;
+  if (c.vblocks == 0) c.splits = 1;
+  // A step whose class of 1-16 columns and whose tiles both hold sequences runs the two in one launch
+  // (mixed_step_kernel), when the host knows the class's count (its grid then holds exactly its work
+  // items), the split counts are the library's and the class's split states fit behind the tiles' (in
+  // the launch of their own they are the workspace's first bytes, which the pre-pass writes here).
+  c.mixed = false;
+  if (c.short_on_decode && c.host.known && c.host.any_tile && c.host.class_n[0] > 0 && c.tile.waves == 4 &&
+      a->num_splits == 0 && c.vblocks > 0) {
+    const int64_t used = (c.v16_bytes + tile_split_bytes(a, c.tile, c.splits) + 15) / 16 * 16;
+    if (const int32_t st = plan_short_rows(a, seg, group, 0, 16, c.host.class_n[0], nullptr, int64_t{1} << 62, c.rows16))
+      return st;
+    const int64_t room = std::max<int64_t>(0, a->workspace_bytes - used);
+    c.mixed = !c.rows16.empty && (c.rows16.p.splits == 1 || c.rows16.state_bytes <= room);
+    if (c.mixed && c.rows16.p.splits > 1) {
+      if (const int32_t st = plan_short_rows(a, seg, group, 0, 16, c.host.class_n[0],
+                                             static_cast<uint8_t*>(a->workspace) + used, room, c.rows16))
         return st;
     }
-    if (max_cols <= 64 || (hp.known && !hp.any_tile)) return LKV_OK;
   }
+  // Workgroups of 8 waves whose two halves take a key half each and merge in LDS, in place of 4-wave tiles
+  // with key splits:
+  // - a grid of at most half the CUs takes as many splits as leave one such workgroup per CU, each in two
+  //   halves (two waves per SIMD where 4-wave tiles leave one): one sequence's 20 tokens at 2K 56.8 -> 30.8
+  //   us, 200 at 5K 51.4 -> 44.4, 40 at 5K (paged) 84.4 -> 41.3, 150 tokens of 8 heads without groups at 16K
+  //   102 -> 84 (with splits that may start in the local segment, effective_splits);
+  // - else an even number of splits runs as pairs, when half as many workgroups still fill the CUs (more than
+  //   7/8 of the rounds they take): the states' round trip through memory and, for 2 splits, the merge
+  //   launch go.  1024 tokens at 7K (256 tiles, 2 splits) 152.4 -> 136 us, 1000 at 3K 127.5 -> 116.0, 512 at
+  //   8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line two sequences' 300 at 3K (160 tiles, 4 splits: 320
+  //   workgroups, a second round of 64) would take 81.6 instead of 78.0, six of 100 at 5K (384) 128.9 of 116.
+  // Uniform calls only: a ragged call's tiles keep one arithmetic whether or not they share a launch with
+  // decode rows.
+  c.halves = false;
+  if (c.tile.waves == 4 && c.splits > 1 && !ragged) {
+    const int64_t half_wgs = c.tile.wgs * c.splits / 2;
+    if (2 * c.tile.wgs <= cus && c.vblocks >= 2 * c.splits * kMinSplitBlocks) {
+      c.splits = static_cast<int>(std::min<int64_t>(c.splits, cus / c.tile.wgs));
+      c.halves = true;
+    } else if (c.splits % 2 == 0 && half_wgs >= cus && half_wgs * 8 > (half_wgs + cus - 1) / cus * cus * 7) {
+      c.splits /= 2;
+      c.halves = true;
+    }
+  }
+  return LKV_OK;
+}
+
+}  // namespace
+
+extern "C" int32_t lkv_prefill_plan(const lkv_prefill_args* a, lkv_prefill_plan_info* info) {
+  using namespace lkv;
+  LKV_REQUIRE(info != nullptr, "null info");
+  SegParams seg;
+  if (const int32_t st = check_prefill_args(a, seg)) return st;
+  *info = lkv_prefill_plan_info{};
+  if (a->batch == 0 || a->tokens == 0) return LKV_OK;
+  CallPlan c;
+  if (const int32_t st = plan_call(a, seg, c)) return st;
+  if (!c.runs_tiles) return LKV_OK;
+  info->tile_waves = c.tile.waves;
+  info->tile_workgroups = c.tile.wgs * c.splits;
+  info->tile_splits = c.splits;
+  info->key_halves = c.halves;
+  info->rows_beside_tiles = c.mixed;
+  return LKV_OK;
+}
+
+extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stream) {
+  using namespace lkv;
+  PrefillParams p;
+  if (const int32_t st = check_prefill_args(a, p.seg)) return st;
+  if (a->batch == 0 || a->tokens == 0) return LKV_OK;
+  CallPlan c;
+  if (const int32_t st = plan_call(a, p.seg, c)) return st;
+  const bool ragged = a->cu_seqlens_q != nullptr;
+  const int group = a->num_q_heads / a->num_kv_heads;
+  // query tokens per sequence (ragged: an upper bound)
+  const int64_t seq_tokens = ragged ? std::min(a->max_seqlen_q, a->tokens) : a->tokens;
+  hipStream_t s = as_stream(stream);
+  if (c.short_on_decode) {  // the decode-kernel classes (with the host copy of the offsets: those that hold a sequence)
+    const int64_t max_cols = seq_tokens * group;
+    const int32_t bounds[4] = {0, 16, 32, 64};
+    for (int i = 0; i < 3; ++i) {
+      if (i == 0 && c.mixed) continue;
+      if (max_cols <= bounds[i]) break;
+      // a uniform call is one class: the one its width falls in
+      if (!ragged && max_cols > bounds[i + 1]) continue;
+      if (c.host.known && c.host.class_n[i] == 0) continue;
+      if (const int32_t st = prefill_on_decode_kernel(a, p.seg, group, bounds[i], bounds[i + 1],
+                                                      c.host.known ? c.host.class_n[i] : -1, s))
+        return st;
+    }
+  }
+  if (!c.runs_tiles) return LKV_OK;
+  const int64_t vblocks = c.vblocks;
   p.q = static_cast<const uint16_t*>(a->q);
   p.q_sb = a->q_stride_b;
   p.q_st = a->q_stride_t;
@@ -1440,41 +1523,14 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
   p.any_wide = reinterpret_cast<float*>(p.vflags + static_cast<int64_t>(a->batch) * a->num_kv_heads * p.vflag_stride);
   p.cu = a->cu_seqlens_q;
   p.rows = a->tokens;
-  p.decode_rows = ragged && short_on_decode ? 64 : -1;
-  const int64_t heads = static_cast<int64_t>(a->num_kv_heads) * a->batch;
-  const int waves = plan.waves;
-  const int64_t tiles = plan.tiles, wgs = plan.wgs;
-  LKV_REQUIRE((mixed ? mixed_grid(rows16.items, wgs * splits) : wgs * splits) < (1LL << 31), "too many query rows");
-  // Workgroups of 8 waves whose two halves take a key half each and merge in LDS, in place of 4-wave tiles
-  // with key splits:
-  // - a grid of at most half the CUs takes as many splits as leave one such workgroup per CU, each in two
-  //   halves (two waves per SIMD where 4-wave tiles leave one): one sequence's 20 tokens at 2K 56.8 -> 30.8
-  //   us, 200 at 5K 51.4 -> 44.4, 40 at 5K (paged) 84.4 -> 41.3, 150 tokens of 8 heads without groups at 16K
-  //   102 -> 84 (with splits that may start in the local segment, effective_splits);
-  // - else an even number of splits runs as pairs, when half as many workgroups still fill the CUs (more than
-  //   7/8 of the rounds they take): the states' round trip through memory and, for 2 splits, the merge
-  //   launch go.  1024 tokens at 7K (256 tiles, 2 splits) 152.4 -> 136 us, 1000 at 3K 127.5 -> 116.0, 512 at
-  //   8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line two sequences' 300 at 3K (160 tiles, 4 splits: 320
-  //   workgroups, a second round of 64) would take 81.6 instead of 78.0, six of 100 at 5K (384) 128.9 of 116.
-  // Uniform calls only: a ragged call's tiles keep one arithmetic whether or not they share a launch with
-  // decode rows.
-  const int64_t cu_count = device_cu_count() > 0 ? device_cu_count() : 256;
-  bool halves = false;
-  if (waves == 4 && splits > 1 && !ragged) {
-    const int64_t half_wgs = wgs * splits / 2;
-    if (2 * wgs <= cu_count && vblocks >= 2 * splits * kMinSplitBlocks) {
-      splits = static_cast<int>(std::min<int64_t>(splits, cu_count / wgs));
-      halves = true;
-    } else if (splits % 2 == 0 && half_wgs >= cu_count &&
-               half_wgs * 8 > (half_wgs + cu_count - 1) / cu_count * cu_count * 7) {
-      splits /= 2;
-      halves = true;
-    }
-  }
+  p.decode_rows = ragged && c.short_on_decode ? 64 : -1;
+  const int splits = c.splits;
+  const int64_t wgs = c.tile.wgs * splits;
+  LKV_REQUIRE((c.mixed ? mixed_grid(c.rows16.items, wgs) : wgs) < (1LL << 31), "too many query rows");
   p.tile_splits = splits;
-  p.ws_o = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(a->workspace) + v16_bytes) : nullptr;
-  p.ws_lse = splits > 1 ? p.ws_o + plan.rows_all * a->num_q_heads * splits * kHeadDim : nullptr;
-  p.tiles = static_cast<int32_t>(tiles);
+  p.ws_o = splits > 1 ? reinterpret_cast<float*>(static_cast<uint8_t*>(a->workspace) + c.v16_bytes) : nullptr;
+  p.ws_lse = splits > 1 ? p.ws_o + c.tile.rows_all * a->num_q_heads * splits * kHeadDim : nullptr;
+  p.tiles = static_cast<int32_t>(c.tile.tiles);
   p.hkv = a->num_kv_heads;
   p.batch = a->batch;
   const bool paged = a->older_block_table != nullptr || a->local_block_table != nullptr;
@@ -1492,23 +1548,25 @@ extern "C" int32_t lkv_prefill_attn(const lkv_prefill_args* a, lkv_stream_t stre
       v16_stage_kernel<false, 1><<<vgrid, 256, 0, s>>>(p);
     if (const int32_t e = check_launch("lkv_prefill_attn (V pre-pass)")) return e;
   }
-  if (mixed) {
-    launch_mixed(paged, wgs * splits, p, rows16, s);
+  if (c.mixed) {
+    launch_mixed(paged, wgs, p, c.rows16, s);
     if (const int32_t e = check_launch("lkv_prefill_attn (decode rows and tiles)")) return e;
-    if (const int32_t e = combine_short_rows(rows16, s, "lkv_prefill_attn (decode rows' merge)")) return e;
+    if (const int32_t e = combine_short_rows(c.rows16, s, "lkv_prefill_attn (decode rows' merge)")) return e;
   } else {
-    launch_tiles(waves, halves, paged, dim3(static_cast<unsigned>(wgs * splits)), p, s);
+    launch_tiles(c.tile.waves, c.halves, paged, dim3(static_cast<unsigned>(wgs)), p, s);
     if (const int32_t e = check_launch("lkv_prefill_attn")) return e;
   }
   if (vblocks == 0) return LKV_OK;
   // the tiles that read a V value of magnitude 65536 or more (flagged by the pre-pass; the instance
   // above skipped them), exactly in bf16, by workgroups that each scan one (sequence, kv head)'s
   // flags at a time
-  launch_wide(waves, paged, static_cast<int>(std::min(heads, cu_count)), p, s);
+  const int64_t heads = static_cast<int64_t>(a->num_kv_heads) * a->batch;
+  const int64_t cus = device_cu_count() > 0 ? device_cu_count() : 256;
+  launch_wide(c.tile.waves, paged, static_cast<int>(std::min(heads, cus)), p, s);
   if (const int32_t e = check_launch("lkv_prefill_attn (wide-range V)")) return e;
   if (splits == 1) return LKV_OK;
-  const int64_t items = plan.rows_all * a->num_q_heads;  // (row, query head) pairs, 4 per workgroup
+  const int64_t items = c.tile.rows_all * a->num_q_heads;  // (row, query head) pairs, 4 per workgroup
   LKV_REQUIRE((items + 3) / 4 < (1LL << 31), "too many query rows");
-  prefill_split_combine_kernel<<<static_cast<unsigned>((items + 3) / 4), 256, 0, s>>>(p, plan.rows_all);
+  prefill_split_combine_kernel<<<static_cast<unsigned>((items + 3) / 4), 256, 0, s>>>(p, c.tile.rows_all);
   return check_launch("lkv_prefill_attn (key-split merge)");
 }

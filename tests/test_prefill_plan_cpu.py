@@ -1,0 +1,81 @@
+"""Which launches lkv_prefill_attn makes for the sequences above 64 query rows per kv head (lkv_prefill_plan),
+by the rules its comments state.  The query reads no device memory, so it runs without a GPU (the library then
+counts 256 CUs, an MI355X's)."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from lastkv_amd import _lib
+
+PTR = 4096  # stands for an aligned device address
+
+
+def plan(lengths, hq=32, hkv=8, older=0, local=0, num_splits=0, tile_waves=0, device_lengths=False, host=True, paged=False,
+         ring=None, room=None):
+    """(waves, splits, halves, mixed) of a call: ``lengths`` an int (one sequence), (batch, tokens) or a list of a
+    ragged call's counts, over ``older`` + ``local`` keys, in the workspace lkv_prefill_workspace_bytes asks for, in
+    that and ``room`` more bytes, or in the smallest (room -1)."""
+
+    lib = _lib.load()
+    a = _lib.PrefillArgs()
+    a.struct_size = ctypes.sizeof(a)
+    ragged = isinstance(lengths, list)
+    B, L = (len(lengths), sum(lengths)) if ragged else lengths if isinstance(lengths, tuple) else (1, lengths)
+    a.batch, a.tokens, a.num_q_heads, a.num_kv_heads, a.head_dim, a.causal = B, L, hq, hkv, 128, 1
+    a.sm_scale = 128 ** -0.5
+    a.q = a.out = PTR
+    a.q_stride_t = a.out_stride_t = hq * 128
+    a.q_stride_b = a.out_stride_b = L * hq * 128
+    a.num_splits, a.tile_waves = num_splits, tile_waves
+    if ragged:
+        cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+        a.cu_seqlens_q, a.max_seqlen_q = PTR, max(lengths)
+        if host:
+            a.cu_seqlens_q_host = cu.ctypes.data
+    blocks = lambda n: -(-n // 32)  # noqa: E731
+    if older:
+        a.older_k = a.older_v = PTR
+        a.older_capacity_tokens, a.older_num_slots, a.older_num_pages = blocks(older) * 32, B, 1
+        a.older_len_const = older
+        if device_lengths:
+            a.older_len = PTR
+    if local:
+        a.local_k = a.local_v = PTR
+        a.local_ring_blocks, a.local_num_slots, a.local_num_pages = blocks(ring or local), B, 1
+        a.local_len_const = local
+        if device_lengths:
+            a.local_len = PTR
+    if paged:
+        for seg, width in (("older", blocks(older)), ("local", blocks(ring or local))):
+            setattr(a, f"{seg}_block_table", PTR)
+            setattr(a, f"{seg}_table_stride", width)
+            setattr(a, f"{seg}_page_stride", 4096)
+    a.workspace = PTR
+    a.workspace_bytes = (lib.lkv_prefill_workspace_min_bytes(ctypes.byref(a)) if room == -1 else
+                         lib.lkv_prefill_workspace_bytes(ctypes.byref(a)) + (room or 0))
+    info = _lib.PrefillPlanInfo()
+    _lib.check(lib.lkv_prefill_plan(ctypes.byref(a), ctypes.byref(info)), "lkv_prefill_plan")
+    return info.tile_waves, info.tile_splits, info.key_halves, info.rows_beside_tiles
+
+
+def test_refused_arguments_are_refused_and_short_calls_have_no_tiles():
+    with pytest.raises(_lib.LastKVNativeError, match="tile_waves"):
+        plan(100, older=1024, tile_waves=3)
+    assert _lib.load().lkv_prefill_plan(None, None) == 1
+    assert plan(16, older=1024) == plan([16, 1, 3], older=1024) == (0, 0, 0, 0)
+
+
+def test_waves_splits_and_the_smallest_workspace():
+    assert plan((4, 1024), older=6144, local=2048) == (8, 1, 0, 0)  # 1024 4-wave tiles
+    assert plan((3, 200), older=2048, local=1024) == (4, 3, 0, 0)  # 168 tiles: three in one round of 512 slots
+    assert plan((3, 200), older=2048, local=1024, room=-1) == (4, 1, 0, 0)
+    assert plan((3, 200), older=2048, local=1024, num_splits=1) == (4, 1, 0, 0)
+    assert plan((3, 200), older=64, local=1024) == (4, 1, 0, 0)  # no equal split starts inside two older blocks
+    assert plan((3, 200), local=1024) == (4, 3, 0, 0)
+    assert plan(20, older=2048, local=1024) == (4, 4, 1, 0)  # 8 tiles: four splits of two halves
+    assert plan(512, older=6144, local=1024) == (4, 2, 1, 0)  # 128 tiles
+    assert plan(512, older=6144, local=1024, device_lengths=True, paged=True) == (4, 2, 1, 0)
