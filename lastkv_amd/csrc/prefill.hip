@@ -1432,11 +1432,13 @@ int32_t plan_call(const lkv_prefill_args* a, const lkv::SegParams& seg, CallPlan
   //   halves (two waves per SIMD where 4-wave tiles leave one): one sequence's 20 tokens at 2K 56.8 -> 30.8
   //   us, 200 at 5K 51.4 -> 44.4, 40 at 5K (paged) 84.4 -> 41.3, 150 tokens of 8 heads without groups at 16K
   //   102 -> 84 (with splits that may start in the local segment, effective_splits);
-  // - else an even number of splits runs as pairs, when half as many workgroups still fill the CUs (more than
-  //   7/8 of the rounds they take): the states' round trip through memory and, for 2 splits, the merge
-  //   launch go.  1024 tokens at 7K (256 tiles, 2 splits) 152.4 -> 136 us, 1000 at 3K 127.5 -> 116.0, 512 at
-  //   8K (128 tiles, 4 splits) 98.5 -> 95.9; past the line two sequences' 300 at 3K (160 tiles, 4 splits: 320
-  //   workgroups, a second round of 64) would take 81.6 instead of 78.0, six of 100 at 5K (384) 128.9 of 116.
+  // - else an even number of splits runs as pairs, when the pairs fill more than 7/8 of the rounds of one
+  //   workgroup per CU that they take (on 256 CUs: 225 to 256 tiles of 2 splits): the states' round trip
+  //   through memory and, for 2 splits, the merge launch go.  One sequence, 2 splits -> pairs: 1024 tokens at 7K
+  //   (256 tiles) 152.4 -> 136 us, 992 (248) 145.4 -> 134.6, 928 (232) 141.1 -> 130.2, 928 at 2K 68.2 -> 57.5; two
+  //   of 470 at 5K (paged, 240) 121 -> 108.6; 12 heads without groups, 2560 at 4K (240) 127.7 -> 117.8.  Past the
+  //   line two sequences' 300 at 3K (160 tiles, 4 splits: 320 workgroups, a second round of 64) would take 81.6
+  //   instead of 78.0, six of 100 at 5K (384) 128.9 of 116.
   // Uniform calls only: a ragged call's tiles keep one arithmetic whether or not they share a launch with
   // decode rows.
   c.halves = false;
@@ -1445,7 +1447,7 @@ int32_t plan_call(const lkv_prefill_args* a, const lkv::SegParams& seg, CallPlan
     if (2 * c.tile.wgs <= cus && c.vblocks >= 2 * c.splits * kMinSplitBlocks) {
       c.splits = static_cast<int>(std::min<int64_t>(c.splits, cus / c.tile.wgs));
       c.halves = true;
-    } else if (c.splits % 2 == 0 && half_wgs >= cus && half_wgs * 8 > (half_wgs + cus - 1) / cus * cus * 7) {
+    } else if (c.splits % 2 == 0 && half_wgs * 8 > (half_wgs + cus - 1) / cus * cus * 7) {
       c.splits /= 2;
       c.halves = true;
     }

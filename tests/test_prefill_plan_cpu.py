@@ -79,3 +79,16 @@ def test_waves_splits_and_the_smallest_workspace():
     assert plan(20, older=2048, local=1024) == (4, 4, 1, 0)  # 8 tiles: four splits of two halves
     assert plan(512, older=6144, local=1024) == (4, 2, 1, 0)  # 128 tiles
     assert plan(512, older=6144, local=1024, device_lengths=True, paged=True) == (4, 2, 1, 0)
+
+
+@pytest.mark.parametrize("lengths,hq,hkv,tiles,pairs", [
+    ((1, 896), 32, 8, 224, 0), ((1, 900), 32, 8, 232, 1), ((1, 928), 32, 8, 232, 1), ((1, 1024), 32, 8, 256, 1),
+    ((2, 470), 32, 8, 240, 1), ((1, 2560), 12, 12, 240, 1), ((3, 160), 64, 8, 240, 1), ((1, 1024), 28, 4, 224, 0),
+    ((1, 480), 64, 8, 240, 1)])
+def test_two_splits_run_as_pairs_when_they_fill_the_round(lengths, hq, hkv, tiles, pairs):
+    """Grids of 224 to 256 tiles take two key splits (512 workgroup slots); as pairs in one workgroup each when
+    that fills more than 7/8 of 256 CUs, at any split of the tiles over sequences and heads."""
+
+    for kw in (dict(older=4096, local=lengths[1]), dict(older=4096, local=3000, device_lengths=True, paged=True)):
+        got = plan(lengths, hq=hq, hkv=hkv, **kw)
+        assert got == ((4, 1, 1, 0) if pairs else (4, 2, 0, 0)), (tiles, got)
