@@ -111,20 +111,6 @@ __global__ __launch_bounds__(kCombineThreads) void decode_combine_kernel(const D
               p.lse != nullptr ? p.lse + bh : nullptr, h / p.group, sm_w, sm_red);
 }
 
-// Key tokens a call can read per sequence (lengths read from device memory bounded by the
-// capacities); Args is lkv_decode_args or lkv_prefill_args (same segment fields).
-template <typename Args>
-int64_t call_key_tokens(const Args* a) {
-  const int64_t ring_tokens = static_cast<int64_t>(a->local_ring_blocks) * kBlockTokens;
-  const int64_t older = a->older_k == nullptr ? 0
-                                              : (a->older_len != nullptr ? a->older_capacity_tokens
-                                                                         : std::min(a->older_len_const, a->older_capacity_tokens));
-  const int64_t local = a->local_k == nullptr
-                            ? 0
-                            : (a->local_len != nullptr ? ring_tokens : std::min<int64_t>(a->local_len_const, ring_tokens));
-  return std::max<int64_t>(older, 0) + std::max<int64_t>(local, 0);
-}
-
 // Non-temporal K/V loads when a call's K/V exceed 384 MiB (more than the 256 MB last-level cache
 // could keep for the next layer's call over the same shared cache); hint 1 / 2 force a policy.
 bool use_nontemporal(int32_t hint, int64_t kv_bytes) { return hint == 2 || (hint == 0 && kv_bytes > (int64_t{384} << 20)); }

@@ -1,6 +1,8 @@
 // Split-K shared-KV decode attention, device side (decode.hip's header comment has the scheme): shared by
 // the decode kernels and by the mixed-step kernel that runs decode rows beside prefill tiles.
 #pragma once
+#include <algorithm>
+
 #include "attn_common.h"
 #include "common.h"
 #include "runtime.h"
@@ -444,6 +446,20 @@ __device__ __attribute__((always_inline)) inline void decode_split_body(const De
       }
     }
   }
+}
+
+// Key tokens a call can read per sequence (lengths read from device memory bounded by the
+// capacities); Args is lkv_decode_args or lkv_prefill_args (same segment fields).
+template <typename Args>
+inline int64_t call_key_tokens(const Args* a) {
+  const int64_t ring_tokens = static_cast<int64_t>(a->local_ring_blocks) * kBlockTokens;
+  const int64_t older = a->older_k == nullptr ? 0
+                                              : (a->older_len != nullptr ? a->older_capacity_tokens
+                                                                         : std::min(a->older_len_const, a->older_capacity_tokens));
+  const int64_t local = a->local_k == nullptr
+                            ? 0
+                            : (a->local_len != nullptr ? ring_tokens : std::min<int64_t>(a->local_len_const, ring_tokens));
+  return std::max<int64_t>(older, 0) + std::max<int64_t>(local, 0);
 }
 
 // The launch of a ragged or short prefill call's sequences of one column class (col_lo < group * tokens <=

@@ -1194,6 +1194,7 @@ struct HostPlan {
   bool known;
   int32_t class_n[3];
   bool any_tile;
+  int64_t tile_rows;  // query rows per kv head of the sequences with more than 64
 };
 
 HostPlan host_plan(const lkv_prefill_args* a, int64_t group) {
@@ -1207,10 +1208,12 @@ HostPlan host_plan(const lkv_prefill_args* a, int64_t group) {
     const int32_t L = std::min(std::min(std::max(cu[b + 1], s0), a->tokens) - s0, lmax);
     if (L <= 0) continue;
     const int64_t cols = L * group;
-    if (cols > 64)
+    if (cols > 64) {
       h.any_tile = true;
-    else
+      h.tile_rows += cols;
+    } else {
       ++h.class_n[cols <= 16 ? 0 : cols <= 32 ? 1 : 2];
+    }
   }
   return h;
 }
@@ -1336,7 +1339,6 @@ int32_t check_prefill_args(const lkv_prefill_args* a, lkv::SegParams& seg) {
   LKV_REQUIRE(a->head_dim == kHeadDim, "head_dim must be 128, got %d", a->head_dim);
   LKV_REQUIRE(a->batch >= 0 && a->tokens >= 0 && a->num_kv_heads > 0 && a->num_q_heads > 0, "bad sizes");
   LKV_REQUIRE(a->num_q_heads % a->num_kv_heads == 0, "num_q_heads must be a multiple of num_kv_heads");
-  const int group = a->num_q_heads / a->num_kv_heads;
   LKV_REQUIRE(a->causal == 0 || a->causal == 1, "causal must be 0 or 1");
   LKV_REQUIRE(a->tile_waves == 0 || a->tile_waves == 4 || a->tile_waves == 8, "tile_waves must be 0, 4 or 8, got %d",
               a->tile_waves);
@@ -1371,6 +1373,26 @@ int32_t check_prefill_args(const lkv_prefill_args* a, lkv::SegParams& seg) {
               static_cast<long long>(a->workspace_bytes));
   LKV_REQUIRE((reinterpret_cast<uintptr_t>(a->workspace) & 15) == 0, "workspace must be 16-byte aligned");
   return LKV_OK;
+}
+
+// Whether one launch of the 1-16 column class and the tiles (mixed_step_kernel) takes less time than two.  It saves
+// a launch's ends and fills the last round of either grid, but a decode item shares its CU there and takes
+// longer.  Where the class is one round of unsplit items (no more than CUs: few enough that each would have a CU
+// to itself), the last item ends the call, so it pays only
+// - over few keys, where the launch's ends weigh more (two launches -> one, one layer of 32 query and 8 kv heads,
+//   20 decode rows + 256 tokens: at 1.5K keys 67.3 -> 53.1 us, at 2.5K 87.2 -> 76.3, at 3K 103 -> 103, at 3.5K
+//   116.8 -> 122.2, at 8K 209.4 -> 243.4), or
+// - where decode rows and tiles take about as long alone, whatever the keys: 128 to 288 query rows of tiles per
+//   decode row (17, 24 and 31 rows + 1024 tokens at 8K, 228 to 128: 285.5 -> 281, 312 -> 297, 350 -> 313; 17 and 24
+//   rows of 64 query heads, 455 and 328: 278 -> 299, 298 -> 311; 17, 24 and 28 rows + 512, 114 to 71: 225 -> 239,
+//   256 -> 261.7, 271.5 -> 276; 34 rows of 4 kv heads with groups of 8 + 1024 at 6K, 234: 206 -> 197).
+// More or split items: 9 rows + 256 tokens at 8K 157.5 -> 121 us, 36 rows + 256 tokens 341.6 -> 293, 90 rows + 64
+// tokens at 4K 284 -> 274, 190 rows + 1024 tokens at 8K 1129 -> 1142.
+constexpr int64_t kMixKeys = 3072, kMixRowsMin = 128, kMixRowsMax = 288;
+
+bool mixing_pays(const lkv_prefill_args* a, const HostPlan& host, const lkv::ShortRowsPlan& rows16, int64_t cus) {
+  if (rows16.p.splits > 1 || rows16.items > cus || lkv::call_key_tokens(a) <= kMixKeys) return true;
+  return host.tile_rows >= kMixRowsMin * host.class_n[0] && host.tile_rows <= kMixRowsMax * host.class_n[0];
 }
 
 // What a call with work to do launches, from its checked arguments.
@@ -1408,10 +1430,12 @@ int32_t plan_call(const lkv_prefill_args* a, const lkv::SegParams& seg, CallPlan
   c.splits = c.tile.splits;
   while (c.splits > 1 && c.v16_bytes + tile_split_bytes(a, c.tile, c.splits) > a->workspace_bytes) --c.splits;
   if (c.vblocks == 0) c.splits = 1;
-  // A step whose class of 1-16 columns and whose tiles both hold sequences runs the two in one launch
+  // A step whose class of 1-16 columns and whose tiles both hold sequences can run the two in one launch
   // (mixed_step_kernel), when the host knows the class's count (its grid then holds exactly its work
   // items), the split counts are the library's and the class's split states fit behind the tiles' (in
-  // the launch of their own they are the workspace's first bytes, which the pre-pass writes here).
+  // the launch of their own they are the workspace's first bytes, which the pre-pass writes here;
+  // lkv_prefill_workspace_bytes counts them there only, so a class with many key splits mixes in a larger
+  // workspace).
   c.mixed = false;
   if (c.short_on_decode && c.host.known && c.host.any_tile && c.host.class_n[0] > 0 && c.tile.waves == 4 &&
       a->num_splits == 0 && c.vblocks > 0) {
@@ -1419,7 +1443,8 @@ int32_t plan_call(const lkv_prefill_args* a, const lkv::SegParams& seg, CallPlan
     if (const int32_t st = plan_short_rows(a, seg, group, 0, 16, c.host.class_n[0], nullptr, int64_t{1} << 62, c.rows16))
       return st;
     const int64_t room = std::max<int64_t>(0, a->workspace_bytes - used);
-    c.mixed = !c.rows16.empty && (c.rows16.p.splits == 1 || c.rows16.state_bytes <= room);
+    c.mixed = !c.rows16.empty && (c.rows16.p.splits == 1 || c.rows16.state_bytes <= room) &&
+              mixing_pays(a, c.host, c.rows16, cus);
     if (c.mixed && c.rows16.p.splits > 1) {
       if (const int32_t st = plan_short_rows(a, seg, group, 0, 16, c.host.class_n[0],
                                              static_cast<uint8_t*>(a->workspace) + used, room, c.rows16))

@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import ctypes
 import os
 import sys
 
@@ -20,6 +21,28 @@ def gpu_available() -> bool:
     import torch
 
     return torch.cuda.is_available()
+
+
+@pytest.fixture
+def prefill_plans(monkeypatch):
+    """The (waves, key splits, halves, decode rows beside the tiles) lkv_prefill_plan gives for every prefill call a
+    test makes (in order; the Python body makes the calls)."""
+
+    from lastkv_amd import _lib, ops
+
+    lib, plans = _lib.load(), []
+    attn = lib.lkv_prefill_attn
+
+    def planned(args, stream):
+        info = _lib.PrefillPlanInfo()
+        _lib.check(lib.lkv_prefill_plan(args, ctypes.byref(info)), "lkv_prefill_plan")
+        plans.append((info.tile_waves, info.tile_splits, info.key_halves, info.rows_beside_tiles))
+        return attn(args, stream)
+
+    monkeypatch.setattr(lib, "lkv_prefill_attn", planned)
+    monkeypatch.setattr(ops, "_host", None)
+    monkeypatch.setattr(ops, "_host_bound", False)
+    return plans
 
 
 def pytest_collection_modifyitems(config, items):

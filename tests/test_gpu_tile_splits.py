@@ -14,13 +14,11 @@ Each test asserts the route its calls take (lkv_prefill_plan).
 
 from __future__ import annotations
 
-import ctypes
-
 import numpy as np
 import pytest
 import torch
 
-from lastkv_amd import _lib, ops
+from lastkv_amd import ops
 from oracle import attention as A
 from oracle import bf16
 
@@ -29,25 +27,6 @@ from test_gpu_varlen import _ragged_case
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
-
-
-@pytest.fixture
-def routes(monkeypatch):
-    """The (waves, key splits, halves) of every prefill call, which the Python body then makes."""
-
-    lib, taken = _lib.load(), []
-    attn = lib.lkv_prefill_attn
-
-    def planned(args, stream):
-        info = _lib.PrefillPlanInfo()
-        _lib.check(lib.lkv_prefill_plan(args, ctypes.byref(info)), "lkv_prefill_plan")
-        taken.append((info.tile_waves, info.tile_splits, info.key_halves))
-        return attn(args, stream)
-
-    monkeypatch.setattr(lib, "lkv_prefill_attn", planned)
-    monkeypatch.setattr(ops, "_host", None)
-    monkeypatch.setattr(ops, "_host_bound", False)
-    return taken
 
 
 def _case(rng, B, Hkv, T0, L, paged):
@@ -88,7 +67,7 @@ def _case(rng, B, Hkv, T0, L, paged):
 @pytest.mark.parametrize("T0", [3000, 70])
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("causal", [True, False])
-def test_key_splits_match_oracle_and_minimum_workspace_runs_unsplit(T0, paged, causal, routes):
+def test_key_splits_match_oracle_and_minimum_workspace_runs_unsplit(T0, paged, causal, prefill_plans):
     rng = np.random.default_rng(11 + 2 * paged + causal + T0)
     B, Hkv, G, L = 1, 2, 4, 512
     seg, k, v = _case(rng, B, Hkv, T0, L, paged)
@@ -112,10 +91,10 @@ def test_key_splits_match_oracle_and_minimum_workspace_runs_unsplit(T0, paged, c
     small = ops.prefill_attention(_t(q), causal=causal, workspace=torch.empty(need, dtype=torch.uint8, device=DEV),
                                   **seg)
     assert torch.equal(small, unsplit)
-    assert routes == [(4, 1, 0) if T0 == 70 else (4, 4, 1), (4, 1, 0), (4, 1, 0)]
+    assert prefill_plans == [(4, 1, 0, 0) if T0 == 70 else (4, 4, 1, 0), (4, 1, 0, 0), (4, 1, 0, 0)]
 
 
-def test_ragged_step_long_row_takes_key_splits(routes):
+def test_ragged_step_long_row_takes_key_splits(prefill_plans):
     """One 300-token row among eleven one-token rows and a 7-token row: the long row's tiles split
     their keys (its older segment is not empty); every row within the bar of the oracle."""
 
@@ -135,7 +114,7 @@ def test_ragged_step_long_row_takes_key_splits(routes):
         got = out[rows].float().cpu().numpy()
         worst = max(worst, A.rel_l2(got, want))
         assert A.max_abs(got, want) <= MAX_ABS and A.rel_l2(got, want) <= REL_L2, f"sequence {b}"
-    assert routes == [(4, 4, 0)]
+    assert prefill_plans == [(4, 4, 0, 0)]
     print(f"ragged step with a long row: worst rel_l2 {worst:.2e}", flush=True)
 
 
@@ -145,7 +124,7 @@ def test_ragged_step_long_row_takes_key_splits(routes):
     (1500, 921, True, False, (4, 1, 1)), (1500, 897, False, True, (4, 1, 1)), (33, 1024, True, False, (4, 1, 0)),
     (-33, 1024, True, False, (4, 1, 1)), (1500, 1024, True, True, (4, 1, 1)), (800, 513, True, False, (4, 3, 0)),
     (800, 512, True, False, (4, 2, 1)), (801, 500, False, False, (4, 2, 1))])
-def test_key_halves_of_one_workgroup_match_oracle(T0, L, causal, wide, route, paged, routes):
+def test_key_halves_of_one_workgroup_match_oracle(T0, L, causal, wide, route, paged, prefill_plans):
     """Uniform calls whose pairs of key splits share a workgroup (226 to 256 tiles of 128 rows: two halves; 126 and
     128 tiles with two splits: two halves of each; 130 tiles take three plain splits): equal and unequal halves, a
     ragged last block, an older segment too short to split (unsplit; with its length on the device, T0 < 0 here,
@@ -165,7 +144,7 @@ def test_key_halves_of_one_workgroup_match_oracle(T0, L, causal, wide, route, pa
     q = _bf(rng, (B, L, Hkv * G, 128))
     lse = torch.empty((B, L, Hkv * G), dtype=torch.float32, device=DEV)
     got = ops.prefill_attention(_t(q), causal=causal, lse=lse, **seg).float()
-    assert routes == [route]
+    assert prefill_plans == [(*route, 0)]
     kt, vt, qt = (torch.from_numpy(np.ascontiguousarray(x)).to(DEV).double() for x in (k[0], v[0], q[0]))
     n = kt.shape[1]
     hide = torch.arange(n, device=DEV)[None, :] > (n - L + torch.arange(L, device=DEV))[:, None]
@@ -183,7 +162,7 @@ def test_key_halves_of_one_workgroup_match_oracle(T0, L, causal, wide, route, pa
 @pytest.mark.parametrize("T0,n1,L,Hkv,G,shift,route", [
     (0, 1200, 100, 2, 4, 0.0, (4, 4, 1)), (0, 1201, 130, 3, 1, 8.0, (4, 4, 1)), (256, 900, 70, 1, 7, 8.0, (4, 4, 1)),
     (640, 1500, 257, 2, 2, 8.0, (4, 4, 1)), (1024, 33, 33, 2, 4, 8.0, (4, 4, 1)), (0, 129, 129, 2, 1, 8.0, (4, 1, 0))])
-def test_key_splits_that_start_in_the_local_segment(T0, n1, L, Hkv, G, shift, route, paged, routes):
+def test_key_splits_that_start_in_the_local_segment(T0, n1, L, Hkv, G, shift, route, paged, prefill_plans):
     """Few tiles over a short (or no) older segment: key splits start in the causal local segment, so some rows see
     no key in a split, row tiles end in padding, and halves get unequal blocks.  With ``shift`` every score sits
     near -90 (2^-130 against a zero reference: a row whose reference were not taken from the first block it sees
@@ -223,7 +202,7 @@ def test_key_splits_that_start_in_the_local_segment(T0, n1, L, Hkv, G, shift, ro
     lse = torch.empty((1, L, Hkv * G), dtype=torch.float32, device=DEV)
     got = ops.prefill_attention(q, causal=True, lse=lse, tile_waves=4, **seg)[0].float()
     # (129 keys: room for one split by the host's lengths, for more by the paged call's capacities)
-    assert routes == [(4, 4, 0) if paged and n1 == 129 else route]
+    assert prefill_plans == [(4, 4, 0, 0) if paged and n1 == 129 else (*route, 0)]
     n = T0 + n1
     hide = torch.arange(n, device=DEV)[None, :] > (n - L + torch.arange(L, device=DEV))[:, None]
     want = torch.empty(L, Hkv * G, 128, dtype=torch.float64, device=DEV)
@@ -239,7 +218,7 @@ def test_key_splits_that_start_in_the_local_segment(T0, n1, L, Hkv, G, shift, ro
 @pytest.mark.parametrize("B,L,T0,tile_waves,route", [
     (1, 40, 1500, 4, (4, 4, 1)), (1, 512, 1500, 0, (4, 2, 1)), (2, 300, 1500, 0, (4, 3, 0)), (1, 130, 0, 4, (4, 3, 0)),
     (1, 900, 1500, 0, (4, 1, 1))])
-def test_a_nan_key_reaches_every_row_that_sees_it(B, L, T0, tile_waves, route, routes):
+def test_a_nan_key_reaches_every_row_that_sees_it(B, L, T0, tile_waves, route, prefill_plans):
     """One NaN key in the local segment: exactly the rows that see it are NaN, with key splits (as halves of a
     workgroup, as states in memory, or both) as without, whichever split holds the key."""
 
@@ -262,10 +241,10 @@ def test_a_nan_key_reaches_every_row_that_sees_it(B, L, T0, tile_waves, route, r
         for splits in (0, 1):
             got = ops.prefill_attention(q, causal=True, tile_waves=tile_waves, num_splits=splits, **seg)
             assert torch.equal(torch.isnan(got), want), f"key {at}, num_splits {splits}"
-            assert routes.pop() == (route if splits == 0 else (4, 1, 0))
+            assert prefill_plans.pop() == ((*route, 0) if splits == 0 else (4, 1, 0, 0))
 
 
-def test_a_split_whose_first_scores_overflow_keeps_its_later_keys(routes):
+def test_a_split_whose_first_scores_overflow_keeps_its_later_keys(prefill_plans):
     """4-wave tiles with key splits, every key range's first block at scores of -infinity (their fp32 sums
     overflow) and all later keys at one finite score of -1.02e33: the output is the mean of V over the later keys, as
     no finite score is lower than the reference of a row that has none yet.  (Every split holds as many keys: in an
@@ -281,6 +260,6 @@ def test_a_split_whose_first_scores_overflow_keeps_its_later_keys(routes):
     ops.pack_kv(k, v, cache)
     # sm_scale log2(e) = 1: the scaled scores are the sums themselves
     got = ops.prefill_attention(q, local=cache, local_len=n, causal=False, sm_scale=float(np.log(2.0)), tile_waves=4)[0].double()
-    assert routes == [(4, 4, 1)]
+    assert prefill_plans == [(4, 4, 1, 0)]
     want = torch.stack([v[0, h // G, ~first].double().mean(0) for h in range(Hkv * G)]).bfloat16().double()[None]
     assert float((got - want).norm() / want.expand_as(got).norm()) <= REL_L2

@@ -233,7 +233,7 @@ def test_ragged_host_offsets_plan_the_same_results(case):
 
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("decode_rows,tile_rows", [(1, [17]), (9, [33, 70]), (70, [100]), (150, [400, 20])])
-def test_ragged_decode_rows_beside_tiles_in_one_launch(decode_rows, tile_rows, paged):
+def test_ragged_decode_rows_beside_tiles_in_one_launch(decode_rows, tile_rows, paged, prefill_plans):
     """With the host copy of the offsets a step's decode rows and tiles run in one launch (decode items and
     tiles interleaved in runs of 64 workgroups): 1 to 150 rows, so fewer and more items than one run, with
     32 splits to one, more and fewer tiles than decode items.  Outputs and LSE equal the separate launches
@@ -254,6 +254,8 @@ def test_ragged_decode_rows_beside_tiles_in_one_launch(decode_rows, tile_rows, p
     for host, ws in ((None, None), (cu, None), (cu, roomy)):
         lse = torch.full((T, Hq), 7.0, dtype=torch.float32, device=DEV)
         results.append((ops.prefill_attention(_t(q), lse=lse, cu_seqlens_q_host=host, workspace=ws, **kw, **seg), lse))
+    one = [p[3] for p in prefill_plans]  # (up to 64 rows take key splits, whose states may need the larger workspace)
+    assert one[0] == 0 and one[2] == 1 and (one[1] == 1 or decode_rows <= 64)
     for out, lse in results[1:]:
         assert torch.equal(out, results[0][0]) and torch.equal(lse, results[0][1])
     for b in (0, decode_rows // 2, len(lengths) - 1):

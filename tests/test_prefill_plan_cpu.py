@@ -92,3 +92,33 @@ def test_two_splits_run_as_pairs_when_they_fill_the_round(lengths, hq, hkv, tile
     for kw in (dict(older=4096, local=lengths[1]), dict(older=4096, local=3000, device_lengths=True, paged=True)):
         got = plan(lengths, hq=hq, hkv=hkv, **kw)
         assert got == ((4, 1, 1, 0) if pairs else (4, 2, 0, 0)), (tiles, got)
+
+
+def _step(rows, tokens, keys=8192, hq=32, hkv=8, **kw):
+    """Whether a step of ``rows`` decode rows and one ``tokens``-token piece over ``keys`` keys (paged, lengths on the
+    device, the recent 2048 in the ring) runs in one launch."""
+
+    return plan([1] * rows + [tokens], hq=hq, hkv=hkv, older=keys - 2048, local=2048, device_lengths=True, paged=True, **kw)[3]
+
+
+@pytest.mark.parametrize("rows,tokens,keys,hq,hkv,one", [
+    (17, 64, 8192, 32, 8, 0), (20, 256, 8192, 32, 8, 0), (31, 512, 8192, 32, 8, 0), (32, 256, 8192, 32, 8, 0),
+    (17, 1024, 8192, 32, 8, 1), (31, 1024, 8192, 32, 8, 1), (32, 1024, 8192, 32, 8, 1), (32, 1023, 8192, 32, 8, 0),
+    (33, 64, 8192, 32, 8, 1), (250, 64, 8192, 32, 8, 1),  # more items than CUs
+    (17, 64, 3072, 32, 8, 1), (17, 64, 3104, 32, 8, 0),  # few keys
+    (17, 1024, 6144, 64, 8, 0), (31, 1024, 6144, 64, 8, 1), (14, 1024, 6144, 12, 12, 0), (22, 1024, 6144, 12, 12, 1)])
+def test_decode_rows_share_the_tiles_launch_where_it_pays(rows, tokens, keys, hq, hkv, one):
+    """One round of unsplit decode items (pairs of row and kv head above half the CUs, at most all of them) shares the
+    launch over few keys or beside tiles of 128 to 288 query rows per decode row, larger classes always."""
+
+    assert _step(rows, tokens, keys, hq, hkv) == one
+    assert _step(rows, tokens, keys, hq, hkv, host=False) == 0  # (the class's size is not known)
+    assert _step(rows, tokens, keys, hq, hkv, num_splits=1) == 0
+    assert _step(rows, tokens, keys, hq, hkv, tile_waves=8) == 0
+
+
+def test_split_decode_rows_share_the_launch_with_room_for_their_states():
+    """Up to half as many items as CUs take key splits: their states must fit behind the tiles'."""
+
+    for rows in (1, 9, 16):
+        assert _step(rows, 256, room=64 << 20) == 1 and _step(rows, 256, room=-1) == 0
