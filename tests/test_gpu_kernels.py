@@ -443,6 +443,19 @@ def test_silu_mul_bit_exact():
     assert torch.equal(got, want)
 
 
+def test_silu_mul_bit_exact_for_every_gate_value():
+    """All 65,536 bf16 gates (zeros, denormals, both sides of -80, infinities, NaN), times 1, a value that rounds, a
+    huge one, zero and an infinity: torch's bits, and NaN where torch has NaN."""
+
+    gate = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.bfloat16).expand(6, -1)
+    up = torch.tensor([1.0, -1.7109375, 3e38, 1e-38, 0.0, float("inf")], device=DEV).bfloat16()[:, None].expand(-1, 65536)
+    got = ops.silu_mul(gate.contiguous(), up.contiguous())
+    want = torch.nn.functional.silu(gate) * up
+    nan = want.isnan()
+    assert torch.equal(got.isnan(), nan) and int(nan.sum()) > 0
+    assert torch.equal(got.view(torch.int16)[~nan], want.contiguous().view(torch.int16)[~nan])
+
+
 @pytest.mark.parametrize("causal", [False, True])
 def test_prefill_lazy_rescale_threshold_regimes(causal):
     """The tile kernel keeps block 0's exact row maximum and rescales only when a later
