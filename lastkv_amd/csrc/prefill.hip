@@ -1118,7 +1118,7 @@ namespace {
 // at most half the CUs, splits each tile's keys over up to 4 workgroups (8-wave tiles: when the call
 // has an older segment) when it leaves the split counts to the library (num_splits 0): a 1024-token
 // piece of one sequence over 8K keys has 256 4-wave tiles, one wave per SIMD, and its key splits put a
-// second wave on each.  lkv_prefill_attn then decides whether splits share workgroups.
+// second wave on each.  plan_call then decides whether splits share workgroups.
 struct TilePlan {
   bool runs;          // the tile kernel runs (some sequence has > 64 rows per kv head, or tile_waves)
   int waves;
