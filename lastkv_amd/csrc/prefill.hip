@@ -439,10 +439,11 @@ constexpr int kTileBuf = 1024;     // uint4 per block buffer (16 KiB)
 // that sees none in its split's first block sees none in the split, whose state for it is empty).  Wider tiles
 // as many equal ones as start inside the older segment, whose blocks every row sees (they split only grids of
 // at most half the CUs; starts in the local segment were not measured for them).  So do calls with an older
-// segment of 1 to kMinOlderBlocks - 1 blocks: they give the bits of the unsplit call where no equal split starts
-// inside it, which callers with a short older segment rely on; with splits anywhere, 512 tokens over 70
-// older and 2048 local keys (one sequence, 32 query and 8 kv heads) would take 42 us instead of 53, 64 tokens
-// 29 instead of 52, and calls of less than 600 keys in all the same 16-22.
+// segment of 1 to kMinOlderBlocks - 1 blocks, not for their speed but for their bits: where no equal split starts
+// inside it they equal the unsplit call's, as they did before splits could start elsewhere, and a test holds
+// them to it.  With splits anywhere, 512 tokens over 70 older and 2048 local keys (one sequence, 32 query and 8
+// kv heads) would take 42 us instead of 53, 64 tokens 29 instead of 52, and calls of less than 600 keys in all
+// the same 16-22.
 constexpr int kMinSplitBlocks = 4, kMinOlderBlocks = 8;
 
 __host__ __device__ inline int effective_splits(int S, int nbt, int nb0, int waves) {
