@@ -366,8 +366,20 @@ def test_epilogue_forms_agree_bit_for_bit(rounding):
 # ------------------------------------------------------------------ blend
 @pytest.mark.parametrize("chunk,cidx", [(64, 1), (64, 4), (1024, 2), (4, 3), (12, 5)])
 def test_blend_chunk_bit_exact(chunk, cidx):
+    _check_blend(chunk, cidx, 3)
+
+
+@pytest.mark.parametrize("layers", [1, 2, 4, 5, 8])
+@pytest.mark.parametrize("chunk", [64, 12])
+def test_blend_layer_groups_bit_exact(chunk, layers):
+    """One and two layers run in groups of their own, more in groups of 4, the last one not always full."""
+
+    _check_blend(chunk, 3, layers)
+
+
+def _check_blend(chunk, cidx, layers):
     rng = np.random.default_rng(chunk + cidx)
-    layers, B, H = 3, 2, 4
+    B, H = 2, 4
     R = ops.ring_tokens_for_chunk(chunk)
     start = cidx * chunk
     deep_k, deep_v = _bf(rng, (B, H, start + chunk, 128)), _bf(rng, (B, H, start + chunk, 128))
