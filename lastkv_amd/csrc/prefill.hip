@@ -1157,15 +1157,34 @@ TilePlan tile_plan(const lkv_prefill_args* a) {
   // 4-wave tiles: below two workgroups per CU; 8-wave tiles (one per CU): at most half the CUs busy
   const bool idle = t.waves == 4 ? est < 2 * cus : (t.waves == 8 && est * 2 <= cus);
   if (t.runs && idle && a->num_splits == 0 && (a->older_k != nullptr || t.waves == 4) && est > 0) {
-    // as many splits as run in one round of the CUs' workgroup slots; where that is 2 and leaves an eighth of
-    // them empty, 4 in two rounds (768 tokens of one sequence at 8K, 192 4-wave tiles: 4 splits 134 us, 3
-    // splits 156, 2 splits 147; four sequences' 200 tokens at 3K, 224 tiles: 2 splits 84.6, 4 splits 90.4;
-    // nine of 55 tokens at 4K, 144 tiles: 3 splits 88.4, 4 splits 100.6); a grid of more than half the
-    // slots takes 2 while an eighth of them would stay empty
+    // As many splits as run in one round of the CUs' workgroup slots (two 4-wave ones per CU); where that is 2, a
+    // uniform call takes 4 if those leave each CU at most three quarter tiles (one sequence, 32 query and 8 kv
+    // heads, us with 2 and 4 splits: 768 tokens at 8K, 192 tiles, 146.5 and 133, 800 tokens, 200 tiles, 149.4 and
+    // 154.6; 864 at 3K, 216 tiles, 83.8 and 86.7; 608 at 8K, 152 tiles, 3 splits 111.8, 4 splits 126).  A ragged
+    // call, whose decode rows share the slots, takes 4 where 2 leave an eighth of them empty (10 decode rows + 800
+    // tokens at 8K, 208 tiles, 242 and 212).  A grid of more than half the slots takes 2 while an eighth would
+    // stay empty.
     const int64_t slots = cus * (t.waves == 4 ? 2 : 1);
     const int64_t one = slots / est;
     int64_t n = one;
-    if (one <= 2) n = one * est * 8 >= slots * 7 ? one : 2 * one;
+    if (one == 2 && t.waves == 4 && !ragged)
+      n = 4 * est <= 3 * cus ? 4 : 2;
+    else if (one <= 2)
+      n = one * est * 8 >= slots * 7 ? one : 2 * one;
+    // The states' round trip through memory and the merge (10-15 us for 200 tiles) need enough keys to pay.  The
+    // line, in tiles per key block: 3, and 2.5 where the grid is more than two thirds of the CUs, which splits then
+    // relieve less; 4 from three sequences on and 3.5 from two, whose unsplit tiles share fewer of their keys
+    // through the caches and take longer a block.  Unsplit -> split, us: one sequence's 256 tokens (64 tiles)
+    // over 8 blocks 17.3 -> 21.3, over 22 25.7 -> 23.6; 512 (128) over 16 22.2 -> 28.8, over 44 38 -> 34.8; 544 (136)
+    // over 17 22.8 -> 29.7, over 64 49.2 -> 44.5; 704 (176) over 44 38.6 -> 44.6, over 96 68 -> 62.9; 864 (216) over
+    // 27 28.6 -> 37.6, over 64 49.5 -> 53.4, over 140 94.6 -> 87.5; four sequences' 100 (128) over 22 30.7 -> 34,
+    // over 32 40.6 -> 35; three of 200 (168) over 19 27.3 -> 33.9, over 44 51 -> 42.8; four of 180 (192) over 19
+    // 28.6 -> 42.7, over 64 67.6 -> 61.  Pairs of uniform calls merge in LDS and pay at any length (960 tokens, 240
+    // tiles, over 30 blocks 30.5 -> 29).
+    const bool pairs = !ragged && n == 2 && one == 2 && est * 8 > cus * 7;
+    const int64_t batch = ragged ? 1 : a->batch;
+    const int64_t half_tiles_per_block = est * 3 <= cus * 2 ? (batch >= 3 ? 8 : 6) : (batch >= 2 ? 7 : 5);
+    if (t.waves == 4 && !pairs && v16_blocks(a) * half_tiles_per_block < est * 2) n = 1;
     t.splits = static_cast<int>(std::min<int64_t>(kMaxTileSplits, n));
   }
   if (t.splits > 1 && a->older_len == nullptr && (a->local_k == nullptr || a->local_len == nullptr)) {

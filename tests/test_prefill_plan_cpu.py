@@ -74,11 +74,36 @@ def test_waves_splits_and_the_smallest_workspace():
     assert plan((3, 200), older=2048, local=1024) == (4, 3, 0, 0)  # 168 tiles: three in one round of 512 slots
     assert plan((3, 200), older=2048, local=1024, room=-1) == (4, 1, 0, 0)
     assert plan((3, 200), older=2048, local=1024, num_splits=1) == (4, 1, 0, 0)
-    assert plan((3, 200), older=64, local=1024) == (4, 1, 0, 0)  # no equal split starts inside two older blocks
-    assert plan((3, 200), local=1024) == (4, 3, 0, 0)
+    assert plan((3, 200), older=64, local=2048) == (4, 1, 0, 0)  # no equal split starts inside two older blocks
+    assert plan((3, 200), local=2048) == (4, 3, 0, 0)
     assert plan(20, older=2048, local=1024) == (4, 4, 1, 0)  # 8 tiles: four splits of two halves
     assert plan(512, older=6144, local=1024) == (4, 2, 1, 0)  # 128 tiles
     assert plan(512, older=6144, local=1024, device_lengths=True, paged=True) == (4, 2, 1, 0)
+
+
+@pytest.mark.parametrize("tokens,tiles,splits", [(544, 136, 3), (672, 168, 3), (704, 176, 4), (768, 192, 4), (800, 200, 2),
+                                                 (896, 224, 2)])
+def test_split_counts_of_one_round(tokens, tiles, splits):
+    """Over 8K keys: as many splits as fit 512 slots, 4 instead of 2 while those are three workgroups a CU; a ragged
+    call (with the decode rows' padding of the grid out of the count) 4 instead of 2 up to 223 tiles."""
+
+    assert plan(tokens, older=6144, local=2048) == (4, splits, 0, 0)
+    assert plan([tokens], older=6144, local=2048)[:3] == (4, 4 if 171 <= tiles < 224 else splits, 0)
+
+
+@pytest.mark.parametrize("lengths,blocks,tiles", [((1, 160), 14, 40), ((1, 256), 22, 64), ((1, 512), 43, 128),
+                                                  ((1, 672), 56, 168), ((1, 704), 71, 176), ((1, 864), 87, 216),
+                                                  ((1, 896), 90, 224), ([700], 71, 176), ((2, 160), 27, 80), ((2, 360), 55, 192),
+                                                  ((3, 100), 24, 96), ((4, 100), 32, 128), ((3, 200), 42, 168),
+                                                  ((4, 180), 55, 192), ((4, 200), 64, 224)])
+def test_key_splits_need_keys_for_their_states(lengths, blocks, tiles):
+    """Tiles split from one key block per three of them on (per 2.5 above two thirds of the CUs; per four and 3.5 in
+    calls of several sequences); first chunks and short contexts below run unsplit."""
+
+    for n in (blocks - 1, blocks):
+        for kw in ({}, dict(device_lengths=True)):  # (a device length counts as its capacity)
+            got = plan(lengths, local=n * 32, **kw)
+            assert (got[1] > 1) == (n == blocks), (n, got)
 
 
 @pytest.mark.parametrize("lengths,hq,hkv,tiles,pairs", [
