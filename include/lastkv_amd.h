@@ -273,7 +273,8 @@ typedef struct lkv_prefill_args {
   /* Key splits of the sequences that run on the decode kernel (at most 64 query rows per kv head):
    * 0 chooses them from the grid and the workspace, and lets the tile kernel split its tiles' keys
    * (over at most 4 workgroups, with up to two halves in each, merged by LSE) when its grid would leave
-   * CUs idle and the workspace holds the states; n in [1, 1024] fixes n (the workspace must then also hold their split states, which
+   * CUs idle, its keys are many enough and the workspace holds the states; n in [1, 1024] fixes n (the workspace
+   * must then also hold their split states, which
    * lkv_prefill_workspace_bytes includes) and runs the tiles unsplit, so that a caller that fixes
    * the split count gets the same arithmetic whatever the batch. */
   int32_t num_splits;
